@@ -249,7 +249,7 @@ int dispatch_fwd(FwdParams p, const af_fwd_args& a, int waves, void* workspace, 
 }
 
 // fp32 forward: keys rotated once into the workspace with RoPE, then
-// fwd_f32_kernel over 128-row query blocks.
+// fwd_f32_kernel (launch_fwd_f32 sets the query blocks of its grid).
 int dispatch_fwd_f32(const af_fwd_args& a, void* workspace, size_t workspace_bytes, hipStream_t s,
                      const af_blockmask* bm = nullptr) {
   if (a.coverage != nullptr)
@@ -290,8 +290,7 @@ int dispatch_fwd_f32(const af_fwd_args& a, void* workspace, size_t workspace_byt
     p.ks[1] = (int64_t)a.seqlen_kv * D;
     p.ks[0] = (int64_t)a.heads_kv * a.seqlen_kv * D;
   }
-  const dim3 grid((unsigned)p.n_mblocks * (unsigned)(p.B * p.Hq));
-  if (launch_fwd_f32(fp, D, grid, s) != 0) return fail(AF_ERR_UNSUPPORTED, "no fp32 forward for head_dim %d", D);
+  if (launch_fwd_f32(fp, D, s) != 0) return fail(AF_ERR_UNSUPPORTED, "no fp32 forward for head_dim %d", D);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(AF_ERR_LAUNCH, "fp32 forward launch failed: %s", hipGetErrorString(e));
   return AF_OK;

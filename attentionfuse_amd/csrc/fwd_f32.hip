@@ -4,11 +4,33 @@
 
 namespace af {
 
-int launch_fwd_f32(const FwdF32Params& p, int head_dim, dim3 grid, hipStream_t s) {
+template <int D, int KW>
+static int go(const FwdF32Params& p, int blocks, hipStream_t s) {
+  FwdF32Params q = p;
+  q.f.n_mblocks = blocks;
+  hipLaunchKernelGGL((fwd_f32_kernel<D, KW>), dim3((unsigned)(blocks * p.f.B * p.f.Hq)),
+                     dim3((KW > 1 ? KW : kF32Waves) * 64), 0, s, q);
+  return 0;
+}
+
+template <int D>
+static int pick_kw(const FwdF32Params& p, hipStream_t s) {
+  const int blocks32 = (p.f.Nq + 31) / 32;   // of one head
+  switch (f32_key_waves(D, (int64_t)blocks32 * p.f.B * p.f.Hq)) {
+    case 8:
+      if constexpr (D <= 64) return go<D, 8>(p, blocks32, s);
+      return -1;
+    case 4: return go<D, 4>(p, blocks32, s);
+    case 2: return go<D, 2>(p, blocks32, s);
+  }
+  return go<D, 1>(p, (p.f.Nq + kF32BlockM - 1) / kF32BlockM, s);
+}
+
+int launch_fwd_f32(const FwdF32Params& p, int head_dim, hipStream_t s) {
   switch (head_dim) {
-    case 32: hipLaunchKernelGGL((fwd_f32_kernel<32>), grid, dim3(kF32Waves * 64), 0, s, p); return 0;
-    case 64: hipLaunchKernelGGL((fwd_f32_kernel<64>), grid, dim3(kF32Waves * 64), 0, s, p); return 0;
-    case 128: hipLaunchKernelGGL((fwd_f32_kernel<128>), grid, dim3(kF32Waves * 64), 0, s, p); return 0;
+    case 32: return pick_kw<32>(p, s);
+    case 64: return pick_kw<64>(p, s);
+    case 128: return pick_kw<128>(p, s);
   }
   return -1;
 }

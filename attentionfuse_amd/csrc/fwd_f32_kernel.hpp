@@ -8,7 +8,9 @@
 //
 // Structure.  One wave owns 32 query rows; a workgroup is four independent
 // waves (128 rows of one (b, h_q)), with no barrier after the query rows
-// are staged.  Per 32-key tile a wave computes
+// are staged.  Grids too small to fill the chip put two to eight waves on
+// one 32-row block instead, each with its share of the key tiles
+// (f32_key_waves).  Per 32-key tile a wave computes
 //   S^T (32 keys x 32 queries) = K Q^T   in D/2 MFMAs (K-dim 2 each), and
 //   O^T (D x 32 queries) += V^T P^T      in 16 * D/32 MFMAs.
 // The dot-product order is free, so MFMA i pairs d = i (lanes 0-31) with
@@ -83,17 +85,48 @@ struct F32Vec<4> {
   typedef f32x4 T;
 };
 
-template <int D>
-__global__ void __launch_bounds__(kF32Waves * 64) fwd_f32_kernel(const FwdF32Params P) {
+// Waves that share one 32-row query block (KW below).  A wave's walk is a
+// serial chain of tiles (32 keys: 4096 cycles of MFMA at D = 64, about 4.5 us
+// alone on its SIMD), so while the 32-row blocks do not fill the chip the
+// chain, not the arithmetic, is the time: the keys of a block are then
+// split over 8, 4 or 2 waves, the most whose waves still come to at most 2.25
+// times those resident at once (2 per SIMD at D = 64, 4 at 32, 1 at 128).
+// Measured (us; one wave per block, then 2, 4, 8), causal, D = 64:
+//   12 heads x 512 (192 blocks)    71   37   22   18.5
+//   12 x 1000 (384)               138   79   45   32
+//   48 x 512 (768)                 72   48   39   38
+//   36 x 1024 (1152)              145   98   82   87
+//   72 x 1024 (2304)              176  144  149  166
+//   48 x 2048 (3072)              351  350  340  375
+// and D = 128 (at most 4: a wave takes more than the 256 registers of two
+// per SIMD): 32 x 512 (512 blocks) 104 / 58 / 46, 32 x 1024 (1024) 201 / 122
+// / 140, 64 x 1024 (2048) 238 / 242 / 275.
+inline int f32_key_waves(int D, int64_t blocks32) {
+  const int64_t most = 9216 / (D / 32);
+  for (int kw = D <= 64 ? 8 : 4; kw > 1; kw /= 2)
+    if (blocks32 * kw <= most) return kw;
+  return 1;
+}
+
+// KW = 1: four waves of 32 query rows each.  KW > 1: KW waves on the same 32
+// rows, wave w walking the key tiles w, w + KW, ... with its own running max
+// and sums, merged through LDS at the end.
+template <int D, int KW>
+__global__ void __launch_bounds__((KW > 1 ? KW : kF32Waves) * 64) fwd_f32_kernel(const FwdF32Params P) {
+  constexpr int NW = KW > 1 ? KW : kF32Waves;
+  constexpr int NQB = NW / KW;   // 32-row query blocks of the workgroup
   constexpr int DH = D / 2;   // d per lane half in the score MFMAs
   constexpr int DC = D / 32;  // output column blocks
   constexpr int QP = D + 4;   // LDS row pitch in floats: rows 16 bytes apart in bank order
   typedef typename F32Vec<DC>::T VecC;
-  __shared__ __attribute__((aligned(16))) float qs[kF32Waves][32][QP];
+  // the query rows; after the walk (KW > 1) the waves' O rows
+  __shared__ __attribute__((aligned(16))) float qs[NW][32][QP];
+  __shared__ float red[KW > 1 ? KW : 1][2][32];   // KW > 1: running max and row sum
 
   const FwdParams& p = P.f;
   const int mask = P.mask, bias = P.bias, norm = P.norm;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int wq = KW > 1 ? 0 : w;                  // query block of this wave
   const int col = lane & 31, h = lane >> 5;
   const int nbh = p.B * p.Hq;
   int mb = (int)(blockIdx.x / nbh);
@@ -101,12 +134,12 @@ __global__ void __launch_bounds__(kF32Waves * 64) fwd_f32_kernel(const FwdF32Par
   // causal-type masks: the longest key ranges first
   if (mask == MASK_CAUSAL || mask == MASK_CSW) mb = p.n_mblocks - 1 - mb;
   const int b = bh / p.Hq, hq = bh % p.Hq, hk = hq / p.G;
-  const int q0 = mb * kF32BlockM + w * 32;
+  const int q0 = mb * 32 * NQB + wq * 32;
   const int qrow = q0 + col;
 
-  // ---- query rows (rotated with RoPE) into this wave's LDS rows ------------
+  // ---- query rows (rotated with RoPE) into this block's LDS rows -----------
   const float* qg = reinterpret_cast<const float*>(p.q) + b * p.qs[0] + hq * p.qs[1];
-  for (int idx = lane; idx < 32 * (D / 4); idx += 64) {
+  for (int idx = KW > 1 ? threadIdx.x : lane; idx < 32 * (D / 4); idx += 64 * KW) {
     const int r = idx / (D / 4), c4 = (idx % (D / 4)) * 4;
     const int n = q0 + r;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
@@ -122,7 +155,7 @@ __global__ void __launch_bounds__(kF32Waves * 64) fwd_f32_kernel(const FwdF32Par
         for (int j = 0; j < 4; ++j) v[j] = lo ? v[j] * c[j] - pv[j] * s[j] : v[j] * c[j] + pv[j] * s[j];
       }
     }
-    *reinterpret_cast<f32x4*>(&qs[w][r][c4]) = v;
+    *reinterpret_cast<f32x4*>(&qs[wq][r][c4]) = v;
   }
   __syncthreads();
   if (q0 >= p.Nq) return;
@@ -185,16 +218,17 @@ __global__ void __launch_bounds__(kF32Waves * 64) fwd_f32_kernel(const FwdF32Par
   // cover the load latency, the score MFMAs of each tile waited for their K
   // rows.  One buffer: tile t + 1's rows load while tile t computes.
   constexpr bool kTwoK = AF_F32_TWO_K(D);
-  constexpr int kKAhead = kTwoK ? 2 : 1;
+  constexpr int kKAhead = KW * (kTwoK ? 2 : 1);
+  const int t0 = KW > 1 ? w : 0;                  // this wave's first tile
   f32x4 kva[DH / 4], kvb[kTwoK ? DH / 4 : 1];
   auto load_k = [&](f32x4 (&kv)[DH / 4], int n0) {
     const float* kr = kg + (int64_t)min(n0 + col, p.Nkv - 1) * p.ks[2] + h * DH;
 #pragma unroll
     for (int i = 0; i < DH / 4; ++i) kv[i] = *reinterpret_cast<const f32x4*>(kr + 4 * i);
   };
-  if (ntiles > 0) load_k(kva, tile_n0(0));
+  if (t0 < ntiles) load_k(kva, tile_n0(t0));
   if constexpr (kTwoK) {
-    if (ntiles > 1) load_k(kvb, tile_n0(1));
+    if (t0 + KW < ntiles) load_k(kvb, tile_n0(t0 + KW));
   }
 
   auto tile = [&](int t, f32x4 (&kv)[DH / 4]) __attribute__((always_inline)) {
@@ -210,7 +244,7 @@ __global__ void __launch_bounds__(kF32Waves * 64) fwd_f32_kernel(const FwdF32Par
     for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
     for (int j = 0; j < DH / 4; ++j) {
-      const f32x4 qv = *reinterpret_cast<const f32x4*>(&qs[w][col][h * DH + 4 * j]);
+      const f32x4 qv = *reinterpret_cast<const f32x4*>(&qs[wq][col][h * DH + 4 * j]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[j][e], qv[e], s, 0, 0, 0);
     }
@@ -275,16 +309,65 @@ __global__ void __launch_bounds__(kF32Waves * 64) fwd_f32_kernel(const FwdF32Par
       }
   };
   if constexpr (kTwoK) {
-    for (int t = 0; t < ntiles; t += 2) {
+    for (int t = t0; t < ntiles; t += 2 * KW) {
       tile(t, kva);
-      if (t + 1 < ntiles) tile(t + 1, kvb);
+      if (t + KW < ntiles) tile(t + KW, kvb);
     }
   } else {
-    for (int t = 0; t < ntiles; ++t) tile(t, kva);
+    for (int t = t0; t < ntiles; t += KW) tile(t, kva);
   }
 
   // ---- epilogue: this lane's half of the keys plus its partner's ------------
   const float lt = lsum + xor32(lsum);
+  if constexpr (KW > 1) {
+    // every wave's O row, running max and row sum into LDS; then
+    // O = sum 2^(m_w - M) O_w / sum 2^(m_w - M) l_w, thread by thread (ReLU
+    // rows keep the initial max, so their weights are 1)
+    __syncthreads();                              // the query rows are read
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      VecC st;
+      if constexpr (DC == 1) {
+        st = o[0][r];
+      } else {
+#pragma unroll
+        for (int c = 0; c < DC; ++c) st[c] = o[c][r];
+      }
+      *reinterpret_cast<VecC*>(&qs[w][col][DC * (8 * (r >> 2) + 4 * h + (r & 3))]) = st;
+    }
+    if (h == 0) {
+      red[w][0][col] = m_run;
+      red[w][1][col] = lt;
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < 32 * (D / 4); idx += 64 * KW) {
+      const int r = idx / (D / 4), c4 = (idx % (D / 4)) * 4;
+      const int n = q0 + r;
+      if (n >= p.Nq) break;                       // rows ascend with idx
+      float M = red[0][0][r];
+#pragma unroll
+      for (int i = 1; i < KW; ++i) M = fmaxf(M, red[i][0][r]);
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      float l = 0.f;
+#pragma unroll
+      for (int i = 0; i < KW; ++i) {
+        const float f = __builtin_amdgcn_exp2f(red[i][0][r] - M);
+        l = __builtin_fmaf(f, red[i][1][r], l);
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&qs[i][r][c4]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(f, x[e], acc[e]);
+      }
+      const float inv = (l == 0.f) ? 1.f : 1.f / l;
+      float* orow = reinterpret_cast<float*>(p.o) + b * p.os[0] + hq * p.os[1] + (int64_t)n * p.os[2];
+      *reinterpret_cast<f32x4*>(orow + c4) = acc * inv;
+      if (p.lse != nullptr && c4 == 0) {
+        float L = -INFINITY;
+        if (norm == NORM_SOFTMAX && l > 0.f) L = (M + __log2f(l)) * kLn2;
+        p.lse[b * p.ls[0] + hq * p.ls[1] + (int64_t)n * p.ls[2]] = L;
+      }
+    }
+    return;
+  }
   const float inv = (lt == 0.f) ? 1.f : 1.f / lt;
   if (qrow < p.Nq) {
     float* orow = reinterpret_cast<float*>(p.o) + b * p.os[0] + hq * p.os[1] + (int64_t)qrow * p.os[2];

@@ -66,7 +66,7 @@ inline int bs_xcd_heads(int BH, int64_t head_bytes) {
 // fp32 forward and fp32 key rotation, defined in fwd_f32.hip; return -1 for
 // a head dim with no instantiation.
 struct FwdF32Params;
-int launch_fwd_f32(const FwdF32Params& p, int head_dim, dim3 grid, hipStream_t s);
+int launch_fwd_f32(const FwdF32Params& p, int head_dim, hipStream_t s);
 struct BwdParams;
 int launch_bwd_f32(BwdParams p, const af_bwd_args& a, hipStream_t s);
 int launch_rope_f32(const float* x, float* out, const float* cs, const float* sn, const int64_t* xs, int64_t rs,

@@ -46,6 +46,18 @@ def test_cross_attention_dense(Nq, Nkv):
     assert run_case("dense", 2, 4, 2, Nq, 64, F32, Nkv=Nkv) <= TOL
 
 
+@pytest.mark.parametrize("H,D,N", [(3, 64, 517), (100, 64, 161), (200, 64, 161), (400, 64, 161), (300, 32, 161),
+                                   (800, 32, 161), (1600, 32, 161), (40, 128, 161), (180, 128, 161), (400, 128, 161)])
+@pytest.mark.parametrize("name", ["rope_causal_alibi", "sw", "relu_causal"])
+def test_waves_per_query_block(name, H, D, N):
+    """Head counts on both sides of every step of the rule that puts 8, 4, 2
+    or 1 waves on a 32-row query block: ragged last tile and block, waves
+    with no visible tile (window, first causal blocks).  Same bound as the
+    other cases: the merge adds a few roundings of 2^-24 to sums of 161."""
+    print(f"[fwd f32] {name} H={H} D={D} N={N}", flush=True)
+    assert run_case(name, 1, H, H, N, D, F32) <= TOL
+
+
 def test_config1_exact_shape():
     """BASELINE config 1 as written -- GPT-2-small causal forward, B=1 H=12
     N=512 D=64 fp32, Q/K/V ~ N(0,1) drawn from seed 0 in that order (the
