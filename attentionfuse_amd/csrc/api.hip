@@ -12,6 +12,7 @@
 #include "bwd_f32_kernel.hpp"
 #include "bwd_launch.hpp"
 #include "fwd_f32_kernel.hpp"
+#include "fwd_keys_kernel.hpp"
 #include "launch.hpp"
 #include "launch_decode.hpp"
 #include "validate.hpp"
@@ -172,13 +173,19 @@ BsFwdWorkspace bs_fwd_workspace(const af_fwd_args& a, const af_blockmask* bm) {
   return w;
 }
 
-// With RoPE, rotate K once into the workspace and point the forward at k~.
-int rotate_keys(FwdParams& p, const af_fwd_args& a, void* workspace, size_t workspace_bytes, hipStream_t s) {
+// With RoPE the caller provides room for k~ (also where the kernel then
+// rotates K itself).
+int check_fwd_workspace(const af_fwd_args& a, const void* workspace, size_t workspace_bytes) {
   const size_t need = fwd_workspace_bytes(a);
-  if (need == 0) return AF_OK;
-  if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))
+  if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)))
     return fail(AF_ERR_WORKSPACE, "forward with RoPE needs a %zu-byte workspace (16-byte aligned), got %zu", need,
                 workspace_bytes);
+  return AF_OK;
+}
+
+// With RoPE, rotate K once into the workspace and point the forward at k~.
+void rotate_keys(FwdParams& p, const af_fwd_args& a, void* workspace, hipStream_t s) {
+  if (fwd_workspace_bytes(a) == 0) return;
   const int D = a.key.head_dim;
   RopeRowsParams r;
   r.x = static_cast<const uint16_t*>(a.k);
@@ -202,7 +209,6 @@ int rotate_keys(FwdParams& p, const af_fwd_args& a, void* workspace, size_t work
   p.ks[2] = D;
   p.ks[1] = (int64_t)a.seqlen_kv * D;
   p.ks[0] = (int64_t)a.heads_kv * a.seqlen_kv * D;
-  return AF_OK;
 }
 
 // Waves (32 query rows each) per forward workgroup for dense / causal /
@@ -217,8 +223,24 @@ int dispatch_fwd(FwdParams p, const af_fwd_args& a, int waves, void* workspace, 
     return fail(AF_ERR_UNSUPPORTED, "a (batch, head) slice of K or V spans 4 GiB or more");
   if (!(p.scale > 0.f) || p.scale == INFINITY)
     return fail(AF_ERR_BAD_ARG, "scale must be positive and finite (got %g)", (double)p.scale);
-  int rc = rotate_keys(p, a, workspace, workspace_bytes, s);
+  int rc = check_fwd_workspace(a, workspace, workspace_bytes);
   if (rc) return rc;
+  // grids too small to fill the chip: the keys of a query block split over
+  // the waves of its workgroup
+  // (its loads address whole slices, rows of the last tile included)
+  const int kw = k.norm == AF_NORM_SOFTMAX && k.bias != AF_BIAS_ADDITIVE && k.mask != AF_MASK_BLOCK_SPARSE &&
+                         slice_fits_u32(p.Nkv + 32, p.ks[2], k.head_dim) &&
+                         slice_fits_u32(p.Nkv + 32, p.vs[2], k.head_dim)
+                     ? fwd_key_waves(k.head_dim, k.mask, (int64_t)((p.Nq + 31) / 32) * p.B * p.Hq)
+                     : 0;
+  if (kw == 0 || !keys_rotates_k(k.head_dim)) rotate_keys(p, a, workspace, s);
+  if (kw > 0) {
+    if (launch_fwd_keys(p, k.dtype, k.head_dim, k.mask, k.bias, k.rope != 0, kw, s) != 0)
+      return fail(AF_ERR_UNSUPPORTED, "no key-split forward for this key");
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(AF_ERR_LAUNCH, "forward launch failed: %s", hipGetErrorString(e));
+    return AF_OK;
+  }
   const dim3 grid((unsigned)p.n_mblocks * (unsigned)(p.B * p.Hq));
   rc = -1;
   const bool f16 = k.dtype == AF_F16;

@@ -45,6 +45,7 @@ UNITS = [
     ("bs_split", "bs_split.hip", []),
     ("bwd", "bwd.hip", []),
     ("fwd_f32", "fwd_f32.hip", []),
+    ("fwd_keys", "fwd_keys.hip", []),
     ("bwd_f32", "bwd_f32.hip", []),
     ("fwd_d256_alt", "fwd_d256_alt.hip", []),
     ("bwd_d256_alt", "bwd_d256_alt.hip", []),

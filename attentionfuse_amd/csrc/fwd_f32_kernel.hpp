@@ -90,7 +90,7 @@ struct F32Vec<4> {
 // alone on its SIMD), so while the 32-row blocks do not fill the chip the
 // chain, not the arithmetic, is the time: the keys of a block are then
 // split over 8, 4 or 2 waves, the most whose waves still come to at most 2.25
-// times those resident at once (2 per SIMD at D = 64, 4 at 32, 1 at 128).
+// times those resident at once (2 per SIMD up to D = 64, 1 at 128).
 // Measured (us; one wave per block, then 2, 4, 8), causal, D = 64:
 //   12 heads x 512 (192 blocks)    71   37   22   18.5
 //   12 x 1000 (384)               138   79   45   32
@@ -100,9 +100,10 @@ struct F32Vec<4> {
 //   48 x 2048 (3072)              351  350  340  375
 // and D = 128 (at most 4: a wave takes more than the 256 registers of two
 // per SIMD): 32 x 512 (512 blocks) 104 / 58 / 46, 32 x 1024 (1024) 201 / 122
-// / 140, 64 x 1024 (2048) 238 / 242 / 275.
+// / 140, 64 x 1024 (2048) 238 / 242 / 275; D = 32, 32 x 1000 (1024): 109 / 65 / 49
+// / 51.
 inline int f32_key_waves(int D, int64_t blocks32) {
-  const int64_t most = 9216 / (D / 32);
+  const int64_t most = D <= 64 ? 4608 : 2304;
   for (int kw = D <= 64 ? 8 : 4; kw > 1; kw /= 2)
     if (blocks32 * kw <= most) return kw;
   return 1;

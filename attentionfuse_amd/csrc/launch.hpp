@@ -34,6 +34,12 @@ AF_DECLARE_FWD(launch_fwd_bf16_d256)
 // fwd_d256_alt.hip with the compiler's default MFMA register form.
 void launch_fwd_bf16_d256_causal_add_relu_rope(const FwdParams& p, dim3 grid, hipStream_t stream);
 
+// Key-split forward of small grids, defined in fwd_keys.hip: dense, causal
+// and windowed softmax with no bias or ALiBi, head dims 32, 64 and 128, kw
+// waves (fwd_key_waves) per 32-row query block.  Returns -1 for a
+// combination it does not hold.
+int launch_fwd_keys(const FwdParams& p, int dtype, int d, int mask, int bias, bool rope, int kw, hipStream_t s);
+
 // rope_rows_kernel launchers, defined next to the forward launchers.
 #define AF_DECLARE_ROPE(NAME) int NAME(const RopeRowsParams& p, hipStream_t stream);
 AF_DECLARE_ROPE(launch_rope_f16_d32)

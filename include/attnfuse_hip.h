@@ -295,7 +295,9 @@ int af_bwd_tile(const af_bwd_args* args, const af_blockmask* bm,
  * accept the subsets documented above), else 0. */
 int af_query(const af_spec_key* key);
 /* Forward tile shape used for the key: query rows per workgroup and keys per
- * stage (the coverage counters are kept per 32 query rows x 64 keys). */
+ * stage (the coverage counters are kept per 32 query rows x 64 keys).  Grids
+ * too small to fill the chip put the waves of a workgroup on one block of 32
+ * query rows instead and split its keys. */
 int af_fwd_tile(const af_spec_key* key, int32_t* block_m, int32_t* block_n);
 
 const char* af_last_error(void);
