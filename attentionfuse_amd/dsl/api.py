@@ -30,6 +30,10 @@ import torch
 
 from ..ir.high_level import (BiasKind, BiasOp, Expr, Graph, MaskKind, MaskOp,
                              NormKind, NormOp, ScoreKind, ScoreOp, TensorSym)
+from ..runtime import autograd as _autograd
+from ..runtime import backward as _backward
+from ..runtime import block_mask as _block_mask
+from ..runtime import dispatch as _dispatch
 from .tracer import trace_attention_fn
 
 
@@ -95,8 +99,12 @@ def relu_attention(scores: Expr) -> Expr:
 
 
 def _wants_grad(*ts) -> bool:
-    return torch.is_grad_enabled() and any(
-        isinstance(t, torch.Tensor) and t.requires_grad for t in ts)
+    if not torch.is_grad_enabled():
+        return False
+    for t in ts:
+        if isinstance(t, torch.Tensor) and t.requires_grad:
+            return True
+    return False
 
 
 def attention(fn: Callable) -> Callable:
@@ -106,7 +114,7 @@ def attention(fn: Callable) -> Callable:
     @functools.wraps(fn)
     def wrapper(Q, K, V, *, bias=None, cos=None, sin=None, block_mask=None,
                 return_graph: bool = False, **kwargs):
-        key = (Q.shape[-1], str(Q.dtype))
+        key = (Q.shape[-1], Q.dtype)
         graph = graphs.get(key)
         if graph is None:
             graph = trace_attention_fn(fn, Q, K, V)
@@ -130,33 +138,29 @@ _INFERENCE_ONLY_KWARGS = ("out", "save_lse", "coverage")
 
 
 def _route(graph: Graph, Q, K, V, bias, cos, sin, block_mask, kwargs):
-    from ..runtime.backward import can_backward
-    masks = {m.kind for m in graph.collect_masks()}
     grad = _wants_grad(Q, K, V)
-    unknown = set(kwargs) - {"alibi_slopes", *_INFERENCE_ONLY_KWARGS}
+    unknown = kwargs and set(kwargs) - {"alibi_slopes", *_INFERENCE_ONLY_KWARGS}
     if unknown:
         raise TypeError(f"unexpected keyword arguments {sorted(unknown)}")
     slopes = kwargs.get("alibi_slopes")
-    autograd = grad and can_backward(graph)
-    if autograd and set(kwargs) & set(_INFERENCE_ONLY_KWARGS):
+    autograd = grad and _backward.can_backward(graph)
+    if autograd and kwargs and set(kwargs) & set(_INFERENCE_ONLY_KWARGS):
         raise ValueError(
             f"{sorted(set(kwargs) & set(_INFERENCE_ONLY_KWARGS))} are not "
             "supported when an input requires grad (the autograd path "
             "allocates its own output and log-sum-exp)")
 
-    if MaskKind.BLOCK_SPARSE in masks:
-        from ..runtime.block_mask import BlockMask, run_block_sparse_graph
+    if MaskKind.BLOCK_SPARSE in graph.mask_kinds():
         if block_mask is None:
             raise RuntimeError(
                 "this graph uses af.block_sparse(); pass block_mask=<BlockMask> "
                 "at call time (build one with "
                 "attnfuse.create_block_mask(predicate, Q_LEN, KV_LEN))")
-        if not isinstance(block_mask, BlockMask):
+        if not isinstance(block_mask, _block_mask.BlockMask):
             raise TypeError("block_mask must be an attnfuse.BlockMask")
         if autograd:
-            from ..runtime.autograd import AttnFuseFunction
-            return AttnFuseFunction.apply(graph, Q, K, V, bias, cos, sin,
-                                          block_mask, slopes)
+            return _autograd.AttnFuseFunction.apply(
+                graph, Q, K, V, bias, cos, sin, block_mask, slopes)
         if grad:
             warnings.warn("AttnFuse: no backward for this block-sparse graph; "
                           "the output carries no gradient", stacklevel=3)
@@ -164,19 +168,17 @@ def _route(graph: Graph, Q, K, V, bias, cos, sin, block_mask, kwargs):
             raise ValueError("coverage= is taken by the dense/causal/windowed "
                              "forward; use runtime.run_block_sparse for "
                              "block-sparse counters")
-        return run_block_sparse_graph(graph, Q, K, V, block_mask, cos=cos,
-                                      sin=sin, out=kwargs.get("out"),
-                                      save_lse=kwargs.get("save_lse"),
-                                      alibi_slopes=slopes)
+        return _block_mask.run_block_sparse_graph(
+            graph, Q, K, V, block_mask, cos=cos, sin=sin,
+            out=kwargs.get("out"), save_lse=kwargs.get("save_lse"),
+            alibi_slopes=slopes)
 
     if grad:
         if autograd:
-            from ..runtime.autograd import AttnFuseFunction
-            return AttnFuseFunction.apply(graph, Q, K, V, bias, cos, sin, None,
-                                          slopes)
+            return _autograd.AttnFuseFunction.apply(
+                graph, Q, K, V, bias, cos, sin, None, slopes)
         warnings.warn("AttnFuse: this graph is outside the backward scope "
                       "(softmax with full/causal/sliding-window/block-sparse "
                       "masks and none/ALiBi bias); the output carries no "
                       "gradient", stacklevel=3)
-    from ..runtime.dispatch import run_attention
-    return run_attention(graph, Q, K, V, bias=bias, cos=cos, sin=sin, **kwargs)
+    return _dispatch.run_attention(graph, Q, K, V, bias=bias, cos=cos, sin=sin, **kwargs)

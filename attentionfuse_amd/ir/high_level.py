@@ -140,6 +140,21 @@ class Graph:
     v: TensorSym
     root: MatMulPV
     _signature: Optional[str] = field(default=None, repr=False)
+    _facts: Optional[dict] = field(default=None, repr=False)
+
+    def fact(self, name: str, compute):
+        """``compute(self)``, remembered under ``name``: like the signature, a
+        property of the traced nodes, which do not change after tracing."""
+        facts = self._facts
+        if facts is None:
+            facts = self._facts = {}
+        if name not in facts:
+            facts[name] = compute(self)
+        return facts[name]
+
+    def mask_kinds(self) -> frozenset:
+        return self.fact("mask_kinds", lambda g: frozenset(
+            m.kind for m in g.collect_masks()))
 
     def walk(self) -> Iterator[tuple]:
         """Pre-order (node, parent) pairs from the root; shared nodes once."""

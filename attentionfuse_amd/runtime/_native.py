@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 import threading
 from pathlib import Path
 
@@ -205,5 +206,25 @@ def strides(t, n: int):
 
 
 def stream_handle(device) -> int:
+    """The raw handle of torch's current stream on ``device`` (a GPU tensor's
+    device carries its index).  Read directly: building a Stream object for it
+    takes 2 us of the 20 a small forward's host path took."""
     import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+_pack16 = struct.Struct("16q").pack_into
+
+
+def pack_strides(args, *tensors) -> None:
+    """The four-entry strides of four (or eight) tensors into consecutive
+    I64x4 fields from ``q_stride`` on (one call per four: a third of the time
+    of a slice assignment per field)."""
+    at = type(args).q_stride.offset
+    for i in range(0, len(tensors), 4):
+        a, b, c, d = tensors[i:i + 4]
+        _pack16(args, at + 32 * i, *a.stride(), *b.stride(), *c.stride(),
+                *d.stride())

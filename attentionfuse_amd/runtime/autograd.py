@@ -10,6 +10,8 @@ from __future__ import annotations
 
 import torch
 
+from . import block_mask as block_mask_mod
+from . import dispatch, kernel_cache
 from .backward import run_backward
 
 
@@ -18,18 +20,15 @@ class AttnFuseFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, graph, Q, K, V, bias, cos, sin, block_mask=None,
                 alibi_slopes=None):
-        from .dispatch import run_attention
-        from .kernel_cache import get_or_compile
         B, Hq, Nq, _ = Q.shape
         L = torch.empty(B, Hq, Nq, dtype=torch.float32, device=Q.device)
-        bundle = get_or_compile(graph)
+        bundle = kernel_cache.get_or_compile(graph)
         if block_mask is not None:
-            from .block_mask import run_block_sparse_graph
-            out = run_block_sparse_graph(graph, Q, K, V, block_mask, cos=cos,
+            out = block_mask_mod.run_block_sparse_graph(graph, Q, K, V, block_mask, cos=cos,
                                          sin=sin, save_lse=L,
                                          alibi_slopes=alibi_slopes)
         else:
-            out = run_attention(graph, Q, K, V, bias=bias, cos=cos, sin=sin,
+            out = dispatch.run_attention(graph, Q, K, V, bias=bias, cos=cos, sin=sin,
                                 save_lse=L, alibi_slopes=alibi_slopes)
         ctx.graph = graph
         ctx.sm_scale = bundle.sm_scale

@@ -19,15 +19,16 @@ _MASK_CODES = {MaskKind.FULL: 0, MaskKind.CAUSAL: 1,
                MaskKind.SLIDING_WINDOW: 2, MaskKind.BLOCK_SPARSE: 3}
 
 
-def can_backward(graph: Graph) -> bool:
+def _backward_graph(graph: Graph) -> bool:
     if graph.norm().kind is not NormKind.SOFTMAX:
         return False
-    masks = {m.kind for m in graph.collect_masks()}
-    if masks - set(_MASK_CODES):
+    if graph.mask_kinds() - set(_MASK_CODES):
         return False
-    if {b.kind for b in graph.collect_biases()} - {BiasKind.ALIBI}:
-        return False
-    return True
+    return not {b.kind for b in graph.collect_biases()} - {BiasKind.ALIBI}
+
+
+def can_backward(graph: Graph) -> bool:
+    return graph.fact("backward", _backward_graph)
 
 
 # Backward launch override, the counterpart of the reference's _BWD_TILE
@@ -123,7 +124,7 @@ def _run_backward_key(key, Q, K, V, O, L, dO, sm_scale, window, cos, sin,
     if L.shape != (B, Hq, Nq) or L.dtype != torch.float32:
         raise ValueError("L must be the (B, H_q, N_q) float32 log-sum-exp")
     Qk, Kk, Vk = kernel_layout(Q), kernel_layout(K), kernel_layout(V)
-    Ok, dOk = kernel_layout(O), kernel_layout(dO.to(Q.dtype))
+    Ok, dOk = kernel_layout(O), kernel_layout(dO if dO.dtype == Q.dtype else dO.to(Q.dtype))
     dQ = torch.empty_like(Qk)
     dK = torch.empty_like(Kk)
     dV = torch.empty_like(Vk)
@@ -138,16 +139,10 @@ def _run_backward_key(key, Q, K, V, O, L, dO, sm_scale, window, cos, sin,
     a.dq, a.dk, a.dv = dQ.data_ptr(), dK.data_ptr(), dV.data_ptr()
     a.cos, a.sin = N.ptr(c), N.ptr(s)
     a.alibi_slopes = N.ptr(slopes)
-    a.q_stride[:] = Qk.stride()
-    a.k_stride[:] = Kk.stride()
-    a.v_stride[:] = Vk.stride()
-    a.o_stride[:] = Ok.stride()
-    a.do_stride[:] = dOk.stride()
-    a.dq_stride[:] = dQ.stride()
-    a.dk_stride[:] = dK.stride()
-    a.dv_stride[:] = dV.stride()
+    N.pack_strides(a, Qk, Kk, Vk, Ok, dOk, dQ, dK, dV)
     a.lse_stride[:] = L.stride()
-    a.rope_stride[:] = N.strides(c, 2)
+    if c is not None:
+        a.rope_stride[:] = c.stride()
     a.batch, a.heads_q, a.heads_kv = B, Hq, Hkv
     a.seqlen_q, a.seqlen_kv = Nq, Nkv
     a.rope_len = 0 if c is None else c.shape[0]
@@ -173,6 +168,5 @@ def run_backward(graph: Graph, Q: torch.Tensor, K: torch.Tensor,
     if not can_backward(graph):
         raise NotImplementedError("graph is outside the backward scope")
     bundle = get_or_compile(graph)
-    key = bundle.key.abi_tuple()
-    return _run_backward_key(key, Q, K, V, O, L, dO, sm_scale, bundle.window,
+    return _run_backward_key(bundle.abi, Q, K, V, O, L, dO, sm_scale, bundle.window,
                              cos, sin, block_mask, alibi_slopes)

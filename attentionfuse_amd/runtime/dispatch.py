@@ -17,6 +17,7 @@ import torch
 
 from ..ir.high_level import Graph, MaskKind
 from . import _native as N
+from .flash_decode import can_use_flash_decode, run_flash_decode
 from .kernel_cache import get_or_compile
 
 _TORCH_DTYPES = {"float16": torch.float16, "bfloat16": torch.bfloat16,
@@ -49,6 +50,17 @@ def alibi_slope_values(n_heads: int) -> list:
 
 
 @functools.lru_cache(maxsize=64)
+def _alibi_slopes_f32(n_heads: int, device: torch.device,
+                      dtype: torch.dtype) -> torch.Tensor:
+    """The slopes rounded to ``dtype``, as fp32 on ``device``.  Rounded on the
+    host and copied with a blocking copy, so the tensor is complete for every
+    stream that uses it (cast on the device per call it was one more launch
+    in front of each ALiBi kernel)."""
+    return (torch.tensor(alibi_slope_values(n_heads), dtype=dtype)
+            .to(torch.float32).to(device))
+
+
+@functools.lru_cache(maxsize=64)
 def _alibi_slopes(n_heads: int, device_str: str, dtype_str: str) -> torch.Tensor:
     """Slopes as a 1-D tensor in the given dtype (the reference keeps them in
     Q's dtype, so the kernels see the rounded values)."""
@@ -63,7 +75,7 @@ def _slopes_f32(H: int, Q: torch.Tensor, override) -> torch.Tensor:
         if s.numel() != H:
             raise ValueError(f"alibi_slopes has {s.numel()} values, need {H}")
         return s.reshape(H).to(torch.float32).contiguous()
-    return _alibi_slopes(H, str(Q.device), str(Q.dtype)).to(torch.float32)
+    return _alibi_slopes_f32(H, Q.device, Q.dtype)
 
 
 # ---------------------------------------------------------------------------
@@ -71,9 +83,12 @@ def _slopes_f32(H: int, Q: torch.Tensor, override) -> torch.Tensor:
 # 16-byte aligned with a unit innermost stride.
 # ---------------------------------------------------------------------------
 def _rows_ok(t: torch.Tensor) -> bool:
-    if t.stride(-1) != 1 or t.data_ptr() % 16:
+    s = t.stride()
+    if s[-1] != 1 or t.data_ptr() % 16:
         return False
-    return all(s % 8 == 0 for s in t.stride()[:-1])
+    if len(s) == 4:
+        return not (s[0] | s[1] | s[2]) & 7
+    return all(x % 8 == 0 for x in s[:-1])
 
 
 def kernel_layout(t: torch.Tensor) -> torch.Tensor:
@@ -103,25 +118,29 @@ def rope_tables(cos, sin, Q: torch.Tensor):
                          f"{tuple(cos.shape)} and {tuple(sin.shape)}")
     if c.device != Q.device or s.device != Q.device:
         raise ValueError("cos/sin must live on Q's device")
-    c = kernel_layout(c.to(Q.dtype))
-    s = kernel_layout(s.to(Q.dtype))
+    if c.dtype != Q.dtype:
+        c = c.to(Q.dtype)
+    if s.dtype != Q.dtype:
+        s = s.to(Q.dtype)
+    c, s = kernel_layout(c), kernel_layout(s)
     return c, s
 
 
 def check_qkv(Q, K, V) -> None:
     if not (Q.is_cuda and K.is_cuda and V.is_cuda):
         raise RuntimeError("AttnFuse requires Q/K/V on a GPU (HIP) device")
-    if Q.dim() != 4 or K.dim() != 4 or V.dim() != 4:
+    qs, ks = Q.shape, K.shape
+    if len(qs) != 4 or len(ks) != 4 or V.dim() != 4:
         raise ValueError("Q, K, V must be 4-D (B, H, N, D)")
-    if K.shape != V.shape:
+    if ks != V.shape:
         raise ValueError(f"K and V must have the same shape; got "
-                         f"{tuple(K.shape)}, {tuple(V.shape)}")
-    if Q.shape[0] != K.shape[0] or Q.shape[3] != K.shape[3]:
+                         f"{tuple(ks)}, {tuple(V.shape)}")
+    if qs[0] != ks[0] or qs[3] != ks[3]:
         raise ValueError(f"Q and K/V must agree on (batch, head_dim); got "
-                         f"Q={tuple(Q.shape)}, K={tuple(K.shape)}")
-    if Q.shape[1] % K.shape[1] != 0:
-        raise ValueError(f"Q heads ({Q.shape[1]}) must be a multiple of KV "
-                         f"heads ({K.shape[1]}) for GQA")
+                         f"Q={tuple(qs)}, K={tuple(ks)}")
+    if qs[1] % ks[1] != 0:
+        raise ValueError(f"Q heads ({qs[1]}) must be a multiple of KV "
+                         f"heads ({ks[1]}) for GQA")
     if not (Q.dtype == K.dtype == V.dtype):
         raise ValueError("Q, K, V must share one dtype")
 
@@ -130,21 +149,24 @@ def fill_fwd_args(a: "N.FwdArgsC", key_tuple, Q, K, V, out, lse, c, s, slopes,
                   bias, coverage, scale: float, window: int) -> None:
     a.key = N.SpecKeyC(*key_tuple)
     a.q, a.k, a.v, a.o = Q.data_ptr(), K.data_ptr(), V.data_ptr(), out.data_ptr()
-    a.lse = N.ptr(lse)
-    a.cos, a.sin = N.ptr(c), N.ptr(s)
-    a.alibi_slopes = N.ptr(slopes)
-    a.bias = N.ptr(bias)
-    a.coverage = N.ptr(coverage)
-    a.q_stride[:] = Q.stride()
-    a.k_stride[:] = K.stride()
-    a.v_stride[:] = V.stride()
-    a.o_stride[:] = out.stride()
-    a.lse_stride[:] = N.strides(lse, 3)
-    a.rope_stride[:] = N.strides(c, 2)
-    a.bias_stride[:] = N.strides(bias, 4)
-    a.batch, a.heads_q, a.seqlen_q = Q.shape[0], Q.shape[1], Q.shape[2]
-    a.heads_kv, a.seqlen_kv = K.shape[1], K.shape[2]
-    a.rope_len = 0 if c is None else c.shape[0]
+    N.pack_strides(a, Q, K, V, out)
+    # a new struct is zero: only what is there is written
+    if lse is not None:
+        a.lse = lse.data_ptr()
+        a.lse_stride[:] = N.strides(lse, 3)
+    if c is not None:
+        a.cos, a.sin = c.data_ptr(), s.data_ptr()
+        a.rope_stride[:] = c.stride()
+        a.rope_len = c.shape[0]
+    if slopes is not None:
+        a.alibi_slopes = slopes.data_ptr()
+    if bias is not None:
+        a.bias = bias.data_ptr()
+        a.bias_stride[:] = bias.stride()
+    if coverage is not None:
+        a.coverage = coverage.data_ptr()
+    a.batch, a.heads_q, a.seqlen_q, _ = Q.shape
+    _, a.heads_kv, a.seqlen_kv, _ = K.shape
     a.scale = float(scale)
     a.window = int(window or 0)
 
@@ -187,8 +209,8 @@ def run_attention(
     B, H, Nq, D = Q.shape
     Nkv = K.shape[2]
 
-    from .flash_decode import can_use_flash_decode, run_flash_decode
-    if save_lse is None and coverage is None and can_use_flash_decode(graph, Q, K):
+    if (Nq == 1 and save_lse is None and coverage is None
+            and can_use_flash_decode(graph, Q, K)):
         if out is None:
             out = torch.empty_like(Q)
         return run_flash_decode(graph, Q, K, V, bundle.sm_scale,
@@ -196,7 +218,7 @@ def run_attention(
                                 alibi_slopes=alibi_slopes)
 
     if Nq != Nkv:
-        masks = {m.kind for m in graph.collect_masks()}
+        masks = graph.mask_kinds()
         if masks - {MaskKind.FULL}:
             raise ValueError(
                 f"cross-attention (N_q={Nq} != N_kv={Nkv}) supports only "
@@ -227,11 +249,13 @@ def run_attention(
     Qk, Kk, Vk = kernel_layout(Q), kernel_layout(K), kernel_layout(V)
     o = out if _rows_ok(out) else torch.empty_like(Q)
     args = N.FwdArgsC()
-    fill_fwd_args(args, bundle.key.abi_tuple(), Qk, Kk, Vk, o, save_lse, c, s,
+    fill_fwd_args(args, bundle.abi, Qk, Kk, Vk, o, save_lse, c, s,
                   slopes, b, coverage, bundle.sm_scale, bundle.window)
-    ws = fwd_workspace(args, Q.device)
-    N.check(N.lib().af_fwd(args, N.ptr(ws), _nbytes(ws),
-                           N.stream_handle(Q.device)))
+    dev = Q.device
+    ws = fwd_workspace(args, dev) if c is not None else None
+    rc = N.lib().af_fwd(args, N.ptr(ws), _nbytes(ws), N.stream_handle(dev))
+    if rc:
+        N.check(rc)
     if o is not out:
         out.copy_(o)
     return out

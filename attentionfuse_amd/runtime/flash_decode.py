@@ -23,19 +23,26 @@ from ..ir.high_level import BiasKind, Graph, MaskKind, NormKind
 from . import _native as N
 
 
-def can_use_flash_decode(graph: Graph, Q: torch.Tensor, K: torch.Tensor) -> bool:
-    if Q.shape[2] != 1 or K.shape[2] < 256:
-        return False
-    if {m.kind for m in graph.collect_masks()} - {MaskKind.FULL}:
+def _decode_graph(graph: Graph) -> bool:
+    if graph.mask_kinds() - {MaskKind.FULL}:
         return False
     if {b.kind for b in graph.collect_biases()} - {BiasKind.ALIBI}:
         return False
-    if graph.has_rope or graph.norm().kind is not NormKind.SOFTMAX:
+    return not graph.has_rope and graph.norm().kind is NormKind.SOFTMAX
+
+
+def can_use_flash_decode(graph: Graph, Q: torch.Tensor, K: torch.Tensor) -> bool:
+    if Q.shape[2] != 1 or K.shape[2] < 256:
+        return False
+    if not graph.fact("decode", _decode_graph):
         return False
     if Q.dtype == torch.float32:
         return Q.shape[-1] in (32, 64, 128)
     return Q.shape[-1] in (32, 64, 128, 256) and Q.dtype in (torch.float16,
                                                               torch.bfloat16)
+
+
+_DTYPE_CODES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 
 
 def _pick_num_splits(B: int, H_q: int, N_kv: int, H_kv: int | None = None,
@@ -66,14 +73,11 @@ def run_flash_decode(graph: Graph, Q: torch.Tensor, K: torch.Tensor,
     slopes = _slopes_f32(H_q, Q, alibi_slopes) if bias_kind == 1 else None
     Qk, Kk, Vk = kernel_layout(Q), kernel_layout(K), kernel_layout(V)
     a = N.DecodeArgsC()
-    dt = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}[Q.dtype]
+    dt = _DTYPE_CODES[Q.dtype]
     a.key = N.SpecKeyC(dt, D, 0, bias_kind, 0, 0)
     a.q, a.k, a.v, a.o = Qk.data_ptr(), Kk.data_ptr(), Vk.data_ptr(), out.data_ptr()
     a.alibi_slopes = N.ptr(slopes)
-    a.q_stride[:] = Qk.stride()
-    a.k_stride[:] = Kk.stride()
-    a.v_stride[:] = Vk.stride()
-    a.o_stride[:] = out.stride()
+    N.pack_strides(a, Qk, Kk, Vk, out)
     a.batch, a.heads_q, a.heads_kv, a.seqlen_kv = B, H_q, H_kv, N_kv
     a.scale = float(sm_scale)
     a.num_splits = S

@@ -30,6 +30,7 @@ class LaunchBundle:
     has_additive_bias: bool
     has_rope: bool
     window: int
+    abi: tuple = ()           # key.abi_tuple()
 
     @property
     def kernel(self) -> SpecKey:   # reference field name
@@ -38,6 +39,9 @@ class LaunchBundle:
 
 def get_or_compile(graph: Graph) -> LaunchBundle:
     sig = graph.signature()
+    hit = _cache.get(sig)
+    if hit is not None:
+        return hit
     with _lock:
         hit = _cache.get(sig)
         if hit is not None:
@@ -56,7 +60,8 @@ def get_or_compile(graph: Graph) -> LaunchBundle:
             key=key, sm_scale=float(key.score_scale),
             block_m=key.config.BLOCK_M, bias_kind=key.bias_code,
             has_additive_bias=key.bias_code == 2,
-            has_rope=bool(key.rope_kind), window=int(key.mask_window or 0))
+            has_rope=bool(key.rope_kind), window=int(key.mask_window or 0),
+            abi=key.abi_tuple())
         _cache[sig] = bundle
         return bundle
 

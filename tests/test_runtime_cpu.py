@@ -134,3 +134,27 @@ def test_missing_library_raises_runtime_error(monkeypatch, tmp_path):
     with pytest.raises(RuntimeError, match="cannot load"):
         N.lib()
     assert N._lib is None                  # nothing half-loaded is cached
+
+
+def test_packed_strides_are_the_tensors_own():
+    """Every stride field of the two argument structs, written in one go,
+    holds its tensor's strides (views of any order, zero strides included)."""
+    from attentionfuse_amd.runtime import _native as N
+    x = torch.zeros(2, 16, 3, 64)
+    views = [x, x.transpose(1, 2), x[:, :1].expand(2, 7, 3, 64), x[:, ::2], x[1:], x.transpose(1, 2)[:, :1],
+             torch.zeros(1, 1, 1, 64), x.permute(2, 1, 0, 3)]
+    names = ["q", "k", "v", "o", "do", "dq", "dk", "dv"]
+    for cls, n in ((N.FwdArgsC, 4), (N.DecodeArgsC, 4), (N.BwdArgsC, 8)):
+        a = cls()
+        N.pack_strides(a, *views[:n])
+        for name, v in zip(names[:n], views):
+            assert tuple(getattr(a, f"{name}_stride")) == v.stride(), (cls.__name__, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_slopes_for_the_kernels_are_the_rounded_ones(dtype):
+    from attentionfuse_amd.runtime.dispatch import _alibi_slopes_f32
+    for H in (1, 8, 12, 33):
+        got = _alibi_slopes_f32(H, torch.device("cpu"), dtype)
+        assert got.dtype == torch.float32
+        assert torch.equal(got, _alibi_slopes(H, "cpu", str(dtype)).float())
