@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "attnfuse_hip.h"
 #include "bs_split.hpp"
@@ -344,7 +345,8 @@ int plan_decode(const af_decode_args* a, size_t max_ws, DecodeParams* out, size_
   if (a->key.bias == AF_BIAS_ALIBI && a->alibi_slopes == nullptr) return fail(AF_ERR_BAD_ARG, "ALiBi needs slopes");
   const int D = a->key.head_dim;
   int S = a->num_splits > 0 ? a->num_splits
-                            : af_decode_num_splits(a->batch, a->heads_q, a->heads_kv, a->seqlen_kv, D);
+                            : af_decode_num_splits(a->batch, a->heads_q, a->heads_kv, a->seqlen_kv,
+                                                   a->key.dtype == AF_F32 ? 4 * D : D);
   // split length rounded up to 32 keys; empty trailing splits are dropped
   int split_len = 0;
   auto trim = [&]() {
@@ -401,8 +403,8 @@ int plan_decode(const af_decode_args* a, size_t max_ws, DecodeParams* out, size_
 // Split + combine of a planned decode call, with its partials at `workspace`.
 int enqueue_decode(DecodeParams& p, const af_decode_args* a, void* workspace, hipStream_t s) {
   const size_t rows = (size_t)p.nsplit * p.B * p.Hq;
-  p.ws_ml = static_cast<float*>(workspace);
-  p.ws_acc = p.ws_ml + 2 * rows;
+  p.ws_acc = static_cast<float*>(workspace);   // first: its rows stay 16-byte aligned
+  p.ws_ml = p.ws_acc + rows * a->key.head_dim;
   const dim3 gs((unsigned)p.nsplit, (unsigned)(p.B * p.Hkv * p.nqc));
   const dim3 gc((unsigned)(p.B * p.Hq));
   if (launch_decode(p, a->key.dtype, a->key.head_dim, a->key.bias, gs, gc, s) != 0)
@@ -544,20 +546,37 @@ size_t af_fwd_blocksparse_workspace_bytes(const af_fwd_args* a, const af_blockma
   return a == nullptr ? 0 : bs_fwd_workspace(*a, bm).total;
 }
 
+// The split count with the least estimated time.  One workgroup alone on its
+// CU streams 128-dim 16-bit keys at 13.2 ns each (8 groups, 4096 keys: 8
+// splits 59 us for 32768 keys); all together reach 5.8 TB/s, less where the
+// last round of workgroups leaves CUs idle (64 groups x 32768 keys: 384
+// workgroups 197.9 us, 256 184.7, 512 182.5); the two add in squares near the
+// crossover.  Each workgroup has its start and merge, and more than one split
+// adds the combine launch, 2 us, and the partials of each (320 groups x 1500
+// keys: 4 splits 50.7 us, 8 56.5).  The four waves take 128 keys a step, so a
+// split counts in whole steps (8 groups x 1024 keys: 8 splits 7.6 us, 4 9.2,
+// 1 13.8; x 256 keys: 1 split 6.2, 2 7.5; x 600 keys: 4 splits 8.2, 8 7.4).
+// fp32 callers pass four times the head dim: twice the bytes, on the VALU.
 int32_t af_decode_num_splits(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen_kv,
                              int32_t head_dim) {
-  (void)head_dim;
   if (batch <= 0 || heads_q <= 0 || heads_kv <= 0 || seqlen_kv <= 0) return 1;
   const int g = heads_q / heads_kv;
-  const int64_t groups = (int64_t)batch * heads_kv * ((g + 15) / 16);
-  // ~512 workgroups: the split kernel keeps two steps of K/V per wave in
-  // flight in 254 VGPRs, so two 4-wave workgroups fit a CU (256 CUs); at
-  // least 256 keys per split.  Measured at config 3: 8 splits (512
-  // workgroups) 180.6 us, 16 splits 186.0 us, 12 splits 183.0 us.
-  int64_t s = (512 + groups - 1) / groups;
-  s = std::min<int64_t>(s, std::max<int64_t>(1, seqlen_kv / 256));
-  s = std::max<int64_t>(1, std::min<int64_t>(s, 256));
-  return (int32_t)s;
+  const double groups = (double)batch * heads_kv * ((g + 15) / 16);
+  const double keys = seqlen_kv, dims = head_dim > 0 ? head_dim : 128;
+  const double bw = groups * keys * dims * 4 / 5.8e6;                  // us
+  const int most = std::max(1, std::min(256, seqlen_kv / 96));
+  int best = 1;
+  double best_t = 0;
+  for (int s = 1; s <= most; s += s < 16 ? 1 : s < 64 ? 4 : 16) {
+    const double per_cu = groups * s / 256, rounds = per_cu < 1 ? 1 : std::ceil(per_cu) / per_cu;
+    const double one = 13.2e-3 * dims * std::ceil(keys / s / 128) * std::ceil(per_cu / 2);
+    const double t = std::sqrt(one * one + bw * bw * rounds * rounds) + 0.2 * per_cu + (s > 1 ? 2.0 + 0.05 * s : 0.0);
+    if (s == 1 || t < best_t) {
+      best = s;
+      best_t = t;
+    }
+  }
+  return best;
 }
 
 size_t af_decode_workspace_bytes(int32_t batch, int32_t heads_q, int32_t head_dim, int32_t num_splits) {

@@ -9,12 +9,13 @@ namespace {
 template <class E, int D, int BIAS>
 void go(const DecodeParams& p, dim3 gs, dim3 gc, hipStream_t s) {
   hipLaunchKernelGGL((decode_split_kernel<E, D, BIAS>), gs, dim3(256), 0, s, p);
-  hipLaunchKernelGGL((decode_combine_kernel<E, D>), gc, dim3(256), 0, s, p);
+  if (p.nsplit > 1) hipLaunchKernelGGL((decode_combine_kernel<E, D>), gc, dim3(256), 0, s, p);
 }
 // fp32: the VALU split kernel, then the combine kernel writing fp32
 template <int D, int BIAS>
 void go_f32(const DecodeParams& p, dim3 gs, dim3 gc, hipStream_t s) {
-  hipLaunchKernelGGL((decode_split_f32_kernel<D, BIAS>), gs, dim3(256), 0, s, p);
+  if (p.G == 1) hipLaunchKernelGGL((decode_split_f32_kernel<D, BIAS, 1>), gs, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((decode_split_f32_kernel<D, BIAS, kF32DecHeads<D>()>), gs, dim3(256), 0, s, p);
   hipLaunchKernelGGL((decode_combine_kernel<F16, D, true>), gc, dim3(256), 0, s, p);
 }
 template <int D>

@@ -17,7 +17,21 @@
 //    keeps its own (m, l, O^T) and the waves merge through LDS at the end;
 //  * S^T = K Q^T on the 16x16x32 MFMA with K read straight from HBM into the
 //    A operand (16-byte loads, no LDS); O^T += V^T P^T on the same MFMA with
-//    V^T written to a per-wave LDS tile; P^T feeds the MFMA from registers.
+//    V rows passed through a per-wave LDS tile, read transposed; P^T feeds
+//    the MFMA from registers;
+//  * a cache that is not split (one workgroup per key/value head fills the
+//    chip, or the cache is short) is finished by its workgroup: no partials
+//    and no combine launch.
+//
+// Bound by HBM for large caches (bf16, B = 8, 8 key/value heads of 128 dims,
+// 32768 keys: 1.07 GB in 181 us, 5.9 TB/s, where a read-only probe peaks at
+// 6.2) and by latency for small ones.  V rows written whole to LDS and read
+// back by transposing reads, vector partials, and a combine that reads all
+// splits' (m, l) at once took one sequence's step (8 key/value heads) from
+// 12.2 to 7.6 us at 1024 keys, 16.4 to 9.2 at 4096, 48.4 to 30.4 at 32768, and
+// 16 x 12 heads of 64 dims x 3001 keys from 39.3 to 31.8 (before, V was
+// written transposed word by word and the (m, l) pairs were read one after the
+// other).
 #pragma once
 
 #include "af_common.hpp"
@@ -30,8 +44,8 @@ struct DecodeParams {
   const uint16_t* v;
   uint16_t* o;
   const float* slopes;
-  float* ws_ml;    // (S, B, Hq, 2) fp32: m (log2 units), l
   float* ws_acc;   // (S, B, Hq, D) fp32: unnormalised accumulator
+  float* ws_ml;    // (S, B, Hq, 2) fp32: m (log2 units), l
   int64_t qs[4], ks[4], vs[4], os[4];
   int32_t B, Hq, Hkv, Nkv, G, nqc, nsplit, split_len;
   float scale;
@@ -45,13 +59,26 @@ struct DecodeParams {
 // V^T A operand uses the same key slots: slot e < 4 -> key 4g + e,
 // slot e >= 4 -> key 16 + 4g + (e - 4).
 
+// LDS chunk (16 bytes) of chunk k of row r of a wave's V tile.  A transposing
+// read takes 8 rows of one 32-byte chunk pair per 32 lanes: XORing the pair
+// with the row spreads them over all 64 banks (rows of 64 and 128 bytes share
+// a bank row four and two at a time).
+template <int D>
+__device__ __forceinline__ int dec_v_chunk(int r, int k) {
+  const int f = D >= 128 ? r & 7 : D == 64 ? (r >> 1) & 3 : (r >> 2) & 1;
+  return k ^ (2 * f);
+}
+
 template <class E, int D, int BIAS>
 __global__ void __launch_bounds__(256) decode_split_kernel(const DecodeParams p) {
   constexpr int KSD = D / 32;      // 32-deep k-steps of K Q^T
   constexpr int DB = D / 16;       // 16-row blocks of O^T
-  constexpr int VTP = 32 + 8;      // V^T tile pitch (elements)
-  constexpr int VT_ELEMS = D * VTP;
-  __shared__ __attribute__((aligned(16))) uint16_t lds[4 * VT_ELEMS];
+  constexpr int VT_ELEMS = 32 * D; // a wave's V tile
+  constexpr int RPV = 512 / D;     // V rows per wave load
+  constexpr int VL = 32 / RPV;     // loads per V tile
+  // the waves' V tiles; after the walk their (m, l) and O
+  constexpr int LDS_BYTES = 4 * VT_ELEMS * 2 > (128 + 64 * D) * 4 ? 4 * VT_ELEMS * 2 : (128 + 64 * D) * 4;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_BYTES];
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, c = lane & 15;
@@ -65,9 +92,10 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const DecodeParams p)
   const int hq = hq0 + c;                  // this lane's query column
   const bool qreal = c < nq;
 
-  const uint16_t* __restrict__ kbase = p.k + b * p.ks[0] + hk * p.ks[1];
-  const uint16_t* __restrict__ vbase = p.v + b * p.vs[0] + hk * p.vs[1];
   const int64_t kstr = p.ks[2], vstr = p.vs[2];
+  const int vrow = lane / (D / 8), vch = lane % (D / 8);
+  const uint16_t* __restrict__ kbase = p.k + b * p.ks[0] + hk * p.ks[1] + c * kstr + 8 * g;
+  const uint16_t* __restrict__ vbase = p.v + b * p.vs[0] + hk * p.vs[1] + vrow * vstr + 8 * vch;
 
   // Q^T as B operand: lane (g, q = c) holds Q[q][32 ks + 8 g .. +7].
   u32x4 qf[KSD];
@@ -89,32 +117,41 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const DecodeParams p)
 #pragma unroll
   for (int db = 0; db < DB; ++db) o[db] = f32x4{};
   float m_run = -INFINITY, l_run = 0.f;
-  uint16_t* vt = lds + w * VT_ELEMS;
-  uint32_t* vt32 = reinterpret_cast<uint32_t*>(vt);
+  uint16_t* vt = reinterpret_cast<uint16_t*>(lds) + w * VT_ELEMS;
+  // LDS element offsets of this lane's V chunk of load i (16-byte writes) and
+  // of its transposing reads: within a 16-lane group, result lane L element i
+  // is element L % 4 of the 8 bytes that lane L / 4 + 4 i addresses, so lane
+  // a + 4 i addresses key row 4 g + i (+ 16 for the second read), dims 4 a.
+  auto v_at = [&](int row, int col) -> int { return row * D + 8 * dec_v_chunk<D>(row, col >> 3) + (col & 7); };
+  const int trow = 4 * g + (c >> 2), tcol = 4 * (c & 3);
 
   // One 32-key step of this wave: K rows (A operand of S^T, keys k0 + 16 kb
-  // + c) and V rows (lane owns keys k0 + 2c, 2c + 1 and 16-byte chunks
-  // g + 4 i) come straight from HBM into registers.
+  // + c) and V rows straight from HBM into registers; only a split's last
+  // step has rows past its end (zeros).
   struct StepRegs {
     u32x4 ka[2][KSD];
-    u32x4 va[D / 32][2];
+    u32x4 va[VL];
   };
   auto load_step = [&](int st, StepRegs& r) {
     const int k0 = s_lo + 32 * st;
+    const uint16_t* kp = kbase + k0 * kstr;
+    const uint16_t* vp = vbase + k0 * vstr;
+    if (k0 + 32 <= s_hi) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      const int n = k0 + 16 * kb + c;
-      const bool ok = n < s_hi;
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int ks = 0; ks < KSD; ++ks)
-        r.ka[kb][ks] = ok ? ld16(kbase + n * kstr + 32 * ks + 8 * g) : u32x4{0, 0, 0, 0};
-    }
+        for (int ks = 0; ks < KSD; ++ks) r.ka[kb][ks] = ld16(kp + 16 * kb * kstr + 32 * ks);
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) {
-      const int dc = g + 4 * i;
-      const int n = k0 + 2 * c;
-      r.va[i][0] = (n < s_hi) ? ld16(vbase + n * vstr + 8 * dc) : u32x4{0, 0, 0, 0};
-      r.va[i][1] = (n + 1 < s_hi) ? ld16(vbase + (n + 1) * vstr + 8 * dc) : u32x4{0, 0, 0, 0};
+      for (int i = 0; i < VL; ++i) r.va[i] = ld16(vp + RPV * i * vstr);
+    } else {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int ks = 0; ks < KSD; ++ks)
+          r.ka[kb][ks] = k0 + 16 * kb + c < s_hi ? ld16(kp + 16 * kb * kstr + 32 * ks) : u32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < VL; ++i)
+        r.va[i] = k0 + RPV * i + vrow < s_hi ? ld16(vp + RPV * i * vstr) : u32x4{0, 0, 0, 0};
     }
   };
   auto compute_step = [&](int st, const StepRegs& r) {
@@ -127,18 +164,9 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const DecodeParams p)
 #pragma unroll
       for (int ks = 0; ks < KSD; ++ks) s[kb] = E::mfma16(r.ka[kb][ks], qf[ks], s[kb]);
     }
-    // V^T into this wave's LDS tile: row d, column = key - k0.
+    // V rows into this wave's LDS tile.
 #pragma unroll
-    for (int i = 0; i < D / 32; ++i) {
-      const int dc = g + 4 * i;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t a = r.va[i][0][e >> 1], bq = r.va[i][1][e >> 1];
-        const uint32_t word = (e & 1) ? ((a >> 16) | (bq & 0xffff0000u))
-                                      : ((a & 0xffffu) | (bq << 16));
-        vt32[((8 * dc + e) * VTP + 2 * c) >> 1] = word;
-      }
-    }
+    for (int i = 0; i < VL; ++i) st16(vt + v_at(RPV * i + vrow, 8 * vch), r.va[i]);
     // Online softmax on this lane's eight keys of query c.
     float x[8];
     float mx = -INFINITY;
@@ -175,9 +203,8 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const DecodeParams p)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
-      const uint16_t* row = vt + (16 * db + c) * VTP + 4 * g;
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(row);
-      const u32x2 hi = *reinterpret_cast<const u32x2*>(row + 16);
+      const u32x2 lo = lds_read_tr16(vt + v_at(trow, 16 * db + tcol));
+      const u32x2 hi = lds_read_tr16(vt + v_at(trow + 16, 16 * db + tcol));
       const u32x4 va4 = {lo[0], lo[1], hi[0], hi[1]};
       o[db] = o[db] * alpha;
       o[db] = E::mfma16(va4, pb, o[db]);
@@ -207,80 +234,105 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const DecodeParams p)
   float* red_m = red;              // [4][16]
   float* red_l = red + 64;         // [4][16]
   float* red_o = red + 128;        // [4][16][D]  (q-major)
-  if (g == 0) {
-    red_m[w * 16 + c] = m_run;
-    red_l[w * 16 + c] = lw;
+  if (qreal) {
+    if (g == 0) {
+      red_m[w * 16 + c] = m_run;
+      red_l[w * 16 + c] = lw;
+    }
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+      *reinterpret_cast<f32x4*>(red_o + (w * 16 + c) * D + 16 * db + 4 * g) = o[db];
   }
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red_o[(w * 16 + c) * D + 16 * db + 4 * g + r] = o[db][r];
   __syncthreads();
-  // 256 threads merge 16 x D outputs.
-  for (int idx = tid; idx < 16 * D; idx += 256) {
-    const int qq = idx / D, d = idx - qq * D;
-    if (qq >= nq) continue;
+  // 256 threads merge the nq x D outputs, four dims each.
+  for (int idx = tid; idx < nq * (D / 4); idx += 256) {
+    const int qq = idx / (D / 4), d = 4 * (idx % (D / 4));
     float mstar = -INFINITY;
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) mstar = fmaxf(mstar, red_m[ww * 16 + qq]);
     const float mu = (mstar == -INFINITY) ? 0.f : mstar;
-    float acc = 0.f, lsum = 0.f;
+    f32x4 acc = f32x4{};
+    float lsum = 0.f;
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) {
       const float f = __builtin_amdgcn_exp2f(red_m[ww * 16 + qq] - mu);
-      acc += f * red_o[(ww * 16 + qq) * D + d];
+      const f32x4 ov = *reinterpret_cast<const f32x4*>(red_o + (ww * 16 + qq) * D + d);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += f * ov[e];
       lsum += f * red_l[ww * 16 + qq];
     }
-    const int64_t row = ((int64_t)split * p.B + b) * p.Hq + hq0 + qq;
-    p.ws_acc[row * D + d] = acc;
-    if (d == 0) {
-      p.ws_ml[2 * row] = mstar;
-      p.ws_ml[2 * row + 1] = lsum;
+    if (p.nsplit == 1) {
+      const float inv = (lsum == 0.f) ? 1.f : 1.f / lsum;
+      uint16_t* orow = p.o + b * p.os[0] + (hq0 + qq) * p.os[1] + d;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) orow[e] = E::one(acc[e] * inv);   // o has no alignment promise
+    } else {
+      const int64_t row = ((int64_t)split * p.B + b) * p.Hq + hq0 + qq;
+      *reinterpret_cast<f32x4*>(p.ws_acc + row * D + d) = acc;
+      if (d == 0) *reinterpret_cast<f32x2*>(p.ws_ml + 2 * row) = f32x2{mstar, lsum};
     }
   }
 }
 
-// Combine: one 256-thread workgroup per (batch, query head).  Thread t owns
-// output dim t % D and the splits s = t / D (mod 256 / D); the partial sums
-// of the split groups meet in LDS.  All loads of a thread are independent,
-// so the kernel is bound by the (L2-resident) workspace reads, not latency.
+// Combine: one 256-thread workgroup per (batch, query head).  Each wave takes
+// the maximum of all splits' m on its own, one per lane; thread t then turns
+// the (m, l) pair of split t into a weight 2^(m_t - m*) in LDS, and a thread
+// sums four output dims over every NG-th split (its loads are independent),
+// the NG sums meeting in LDS.  Read one after the other by every thread, the
+// pairs of 64 splits took most of the kernel.
 template <class E, int D, bool F32OUT = false>
 __global__ void __launch_bounds__(256) decode_combine_kernel(const DecodeParams p) {
-  constexpr int NG = 256 / D;
-  __shared__ float red_acc[NG][D];
-  __shared__ float red_l[NG];
-  const int t = threadIdx.x;
-  const int d = t % D, grp = t / D;
+  constexpr int TPR = D / 4;                  // threads per partial row
+  constexpr int NG = 256 / TPR;
+  __shared__ __attribute__((aligned(16))) float red_acc[NG][D];
+  __shared__ float wt[256];
+  __shared__ float red_l[4];
+  const int t = threadIdx.x, lane = t & 63;
+  const int d = 4 * (t % TPR), grp = t / TPR;
   const int row = blockIdx.x;                 // b * Hq + hq
   const int b = row / p.Hq, hq = row - b * p.Hq;
   const int S = p.nsplit;
   const int64_t plane = (int64_t)p.B * p.Hq;
   float mstar = -INFINITY;
-  for (int s = 0; s < S; ++s) mstar = fmaxf(mstar, p.ws_ml[2 * (s * plane + row)]);
-  const float mu = (mstar == -INFINITY) ? 0.f : mstar;
-  float acc = 0.f, lsum = 0.f;
-#pragma unroll 4
-  for (int s = grp; s < S; s += NG) {
-    const int64_t r = s * plane + row;
-    const float f = __builtin_amdgcn_exp2f(p.ws_ml[2 * r] - mu);
-    lsum += f * p.ws_ml[2 * r + 1];
-    acc += f * p.ws_acc[r * D + d];
-  }
-  red_acc[grp][d] = acc;
-  if (d == 0) red_l[grp] = lsum;
-  __syncthreads();
-  if (grp == 0) {
-    float a = 0.f, l = 0.f;
+  for (int s = lane; s < S; s += 64) mstar = fmaxf(mstar, p.ws_ml[2 * (s * plane + row)]);
 #pragma unroll
-    for (int g2 = 0; g2 < NG; ++g2) {
-      a += red_acc[g2][d];
-      l += red_l[g2];
+  for (int off = 1; off < 64; off <<= 1) mstar = fmaxf(mstar, __shfl_xor(mstar, off, 64));
+  const float mu = (mstar == -INFINITY) ? 0.f : mstar;
+  float lsum = 0.f;
+  f32x4 acc = f32x4{};
+  for (int c0 = 0; c0 < S; c0 += 256) {       // one pass but for explicit split counts
+    if (c0 > 0) __syncthreads();
+    if (c0 + t < S) {
+      const f32x2 ml = *reinterpret_cast<const f32x2*>(p.ws_ml + 2 * ((c0 + t) * plane + row));
+      const float f = __builtin_amdgcn_exp2f(ml[0] - mu);
+      wt[t] = f;
+      lsum += f * ml[1];
     }
-    const float inv = (l == 0.f) ? 1.f : 1.f / l;
+    __syncthreads();
+    const int n = min(256, S - c0);
+#pragma unroll 4
+    for (int s = grp; s < n; s += NG) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(p.ws_acc + ((c0 + s) * plane + row) * D + d);
+      const float f = wt[s];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += f * x[e];
+    }
+  }
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) lsum += __shfl_xor(lsum, off, 64);
+  if (lane == 0) red_l[t >> 6] = lsum;
+  *reinterpret_cast<f32x4*>(&red_acc[grp][d]) = acc;
+  __syncthreads();
+  if (t < D) {
+    const float l = (red_l[0] + red_l[1]) + (red_l[2] + red_l[3]);
+    float a = 0.f;
+#pragma unroll
+    for (int g2 = 0; g2 < NG; ++g2) a += red_acc[g2][t];
+    a *= (l == 0.f) ? 1.f : 1.f / l;
     if constexpr (F32OUT)
-      reinterpret_cast<float*>(p.o)[b * p.os[0] + hq * p.os[1] + d] = a * inv;
+      reinterpret_cast<float*>(p.o)[b * p.os[0] + hq * p.os[1] + t] = a;
     else
-      p.o[b * p.os[0] + hq * p.os[1] + d] = E::one(a * inv);
+      p.o[b * p.os[0] + hq * p.os[1] + t] = E::one(a);
   }
 }
 
@@ -301,10 +353,12 @@ __host__ __device__ constexpr int f32_decode_heads(int D) { return 64 / (D / 8) 
 template <int D>
 constexpr int kF32DecHeads() { return f32_decode_heads(D); }
 
-template <int D, int BIAS>
+// GQ: query heads per workgroup, kF32DecHeads(D), or 1 where every key/value
+// head has one query head (the other slots would repeat it: 4 x 12 heads of 64
+// dims, 4096 keys, 54.6 -> 22.2 us).
+template <int D, int BIAS, int GQ>
 __global__ void __launch_bounds__(256) decode_split_f32_kernel(const DecodeParams p) {
   constexpr int CH = D / 8;                 // dims per lane
-  constexpr int GQ = kF32DecHeads<D>();     // query heads per workgroup
   __shared__ float red[4][GQ][2 + D];
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;

@@ -50,6 +50,12 @@ def _pick_num_splits(B: int, H_q: int, N_kv: int, H_kv: int | None = None,
     return int(N.lib().af_decode_num_splits(B, H_q, H_kv or H_q, N_kv, D))
 
 
+def _split_dims(Q: torch.Tensor) -> int:
+    """Head dim as the split rule weighs it: the fp32 kernel's keys cost four
+    times a 16-bit key of the same head dim."""
+    return Q.shape[-1] * (4 if Q.dtype == torch.float32 else 1)
+
+
 def decode_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """A fresh ``nbytes`` byte buffer from torch's caching allocator, owned
     by the current stream of ``device``."""
@@ -66,7 +72,7 @@ def run_flash_decode(graph: Graph, Q: torch.Tensor, K: torch.Tensor,
     _, H_kv, N_kv, _ = K.shape
     if H_kv != num_heads_kv:
         raise ValueError("num_heads_kv does not match K")
-    S = num_splits or _pick_num_splits(B, H_q, N_kv, H_kv, D)
+    S = num_splits or _pick_num_splits(B, H_q, N_kv, H_kv, _split_dims(Q))
     # the library may drop empty trailing splits; size for the request
     nbytes = int(N.lib().af_decode_workspace_bytes(B, H_q, D, S))
     ws = workspace if workspace is not None else decode_workspace(Q.device, nbytes)

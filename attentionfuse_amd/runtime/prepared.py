@@ -74,7 +74,8 @@ def prepare_decode(graph: Graph, Q, K, V, *, out=None, num_splits: int = 0,
                    alibi_slopes=None) -> tuple:
     """-> (launch, out) for a flash-decoding call with its own workspace."""
     from .dispatch import _rows_ok, _slopes_f32, check_qkv
-    from .flash_decode import _pick_num_splits, can_use_flash_decode
+    from .flash_decode import (_pick_num_splits, _split_dims,
+                               can_use_flash_decode)
     from .kernel_cache import get_or_compile
     check_qkv(Q, K, V)
     if not can_use_flash_decode(graph, Q, K):
@@ -87,7 +88,7 @@ def prepare_decode(graph: Graph, Q, K, V, *, out=None, num_splits: int = 0,
     Hkv, Nkv = K.shape[1], K.shape[2]
     if out is None:
         out = torch.empty_like(Q)
-    S = num_splits or _pick_num_splits(B, Hq, Nkv, Hkv, D)
+    S = num_splits or _pick_num_splits(B, Hq, Nkv, Hkv, _split_dims(Q))
     nbytes = int(N.lib().af_decode_workspace_bytes(B, Hq, D, S))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=Q.device)
     slopes = _slopes_f32(Hq, Q, alibi_slopes) if bundle.bias_kind == 1 else None

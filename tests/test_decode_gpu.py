@@ -128,3 +128,23 @@ def test_decode_long_cache(alibi):
         kw = {"alibi_slopes": _alibi_slopes(Hq, "cpu", "torch.bfloat16").float(), "query_offset": N - 1}
     want = O.naive_attention(Q.cpu(), K.cpu(), V.cpu(), **kw)
     assert (out.float().cpu() - want).abs().max().item() <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("splits", [1, 2, 300])
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+def test_unsplit_and_many_splits_into_unaligned_rows(D, splits):
+    """An unsplit cache is finished by its workgroup, more than 256 splits
+    take the combine's second pass; 17 query heads leave a chunk with one
+    real head; the output rows start at odd elements.  16-bit tolerance of
+    the other cases."""
+    B, Hq, Hkv, N, dtype = 2, 34, 2, 9999, torch.bfloat16
+    print(f"[decode] D={D} splits={splits}", flush=True)
+    Q, K, V = make(B, Hq, Hkv, N, D, dtype, seed=D)
+    buf = torch.zeros(B, Hq, 1, D + 1, device="cuda", dtype=dtype)
+    out = buf[..., 1:]
+    g = dense(Q, K, V, return_graph=True)
+    run_flash_decode(g, Q, K, V, D ** -0.5, 0, Hkv, out, num_splits=splits)
+    torch.cuda.synchronize()
+    want = O.naive_attention(Q.cpu(), K.cpu(), V.cpu())
+    assert (out.float().cpu() - want).abs().max().item() <= TOL[dtype]
+    assert not buf[..., 0].any()
