@@ -512,6 +512,14 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 
 // ---------------------------------------------------------------------------
+// (batch, head) of workgroup i of the BH that share a query block.  The
+// dispatcher hands workgroup g to XCD g % 8; with BH a multiple of 8 each XCD
+// gets BH / 8 consecutive heads, so that the query heads of a GQA group read
+// their K and V through one XCD's L2 instead of through several.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int xcd_head(int i, int BH) { return (BH & 7) ? i : (i & 7) * (BH >> 3) + (i >> 3); }
+
+// ---------------------------------------------------------------------------
 // Work item and (batch, head) of workgroup g of a grid of n_items x BH
 // workgroups.  The dispatcher hands workgroup g to XCD g % 8, so with BH a
 // multiple of 8 the default order (item-major, head-minor) keeps every head

@@ -792,7 +792,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams& p, uint16_t* lds, i
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int BH = p.B * p.Hq;
-  int bh = wg % BH;
+  int bh = xcd_head(wg % BH, BH);
   int mbi = wg / BH;
   if constexpr (kIsBs<MASK>) xcd_head_groups(wg, BH, p.bs_q_rows, p.bs_xcd_heads_q, mbi, bh);
   const bool heavy_last = MASK == MASK_CAUSAL || MASK == MASK_CSW;

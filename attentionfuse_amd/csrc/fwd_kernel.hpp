@@ -167,9 +167,9 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 
   const int BH = p.B * p.Hq;
   // m-block-major order: the heaviest query blocks of every head first.
-  // Workgroup g runs on XCD g % 8, so when B*H is a multiple of 8 each XCD
-  // works on a fixed eighth of the heads, whose K/V stay in its L2.
-  int bh = blockIdx.x % BH;
+  // When B*H is a multiple of 8 each XCD works on a fixed eighth of the heads,
+  // whose K/V stay in its L2.
+  int bh = xcd_head(blockIdx.x % BH, BH);
   int mbi = blockIdx.x / BH;
   if constexpr (kIsBs<MASK>) xcd_head_groups(blockIdx.x, BH, p.n_mblocks, p.bs_xcd_heads, mbi, bh);
   const bool heavy_last = MASK == MASK_CAUSAL || MASK == MASK_CSW;

@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(D 
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, c = lane & 31;
   const int BH = p.B * p.Hq;
-  const int bh = blockIdx.x % BH, mbi = blockIdx.x / BH;
+  const int bh = xcd_head(blockIdx.x % BH, BH), mbi = blockIdx.x / BH;
   // causal-type masks: the longest walks first
   const int mb = (mask == MASK_CAUSAL || mask == MASK_CSW) ? p.n_mblocks - 1 - mbi : mbi;
   const int b = bh / p.Hq, hq = bh - b * p.Hq, hk = hq / p.G;
