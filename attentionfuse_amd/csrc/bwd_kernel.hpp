@@ -205,18 +205,18 @@ __device__ inline void load_operand_rows(u32x4* f, const uint16_t* base, int64_t
   for (int ks = 0; ks < KS; ++ks) f[ks] = ok ? ld16(base + row * rstride + 16 * ks + 8 * h) : u32x4{0, 0, 0, 0};
 }
 
-// Store a transposed 32x32-block gradient accumulator (rows = dims,
-// column = this lane's row `row`) as out[row][d], applying the scale and,
-// with ROPE, the inverse rotation R^T at position `row`.
+// Store a wave's transposed 32x32-block gradient accumulator (rows = dims,
+// column = this lane's row `row` of row0 .. row0 + 31) as out[row][d], through
+// the wave's 32 x D elements of LDS at wl, applying the scale and, with ROPE,
+// the inverse rotation R^T at position `row`.
 template <class E, int D, bool ROPE>
-__device__ inline void store_grad_rows(f32x16* acc, uint16_t* out, int64_t rstride, int row, int nvalid,
-                                       float scale, const uint16_t* cos, const uint16_t* sin, int64_t cstride,
-                                       int h) {
+__device__ inline void store_grad_rows(uint16_t* wl, f32x16* acc, uint16_t* out, int64_t rstride, int row0, int row,
+                                       int nvalid, float scale, const uint16_t* cos, const uint16_t* sin,
+                                       int64_t cstride, int h) {
   constexpr int DB = D / 32;
-  if (row >= nvalid) return;
 #pragma unroll
   for (int db = 0; db < DB; ++db) acc[db] *= scale;
-  if constexpr (ROPE) {
+  if (ROPE && row < nvalid) {
     const uint16_t* cr = cos + row * cstride;
     const uint16_t* sr = sin + row * cstride;
     // register group (db, g) holds dims 32 db + 8 g + 4 h + e; its rotate-half
@@ -246,17 +246,7 @@ __device__ inline void store_grad_rows(f32x16* acc, uint16_t* out, int64_t rstri
         }
       }
   }
-  uint16_t* orow = out + row * rstride;
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d0 = 32 * db + 8 * g + 4 * h;
-      u32x2 w2;
-      w2[0] = E::pack(acc[db][4 * g], acc[db][4 * g + 1]);
-      w2[1] = E::pack(acc[db][4 * g + 2], acc[db][4 * g + 3]);
-      *reinterpret_cast<u32x2*>(orow + d0) = w2;
-    }
+  store_rows_via_lds<E, D>(wl, acc, out, rstride, row0, nvalid);
 }
 
 // fp32 row of a transposed 32x32-block accumulator (rows = dims, column =
@@ -753,8 +743,10 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdParams& p, uint16_t* lds, 
     }
     return;
   }
-  store_grad_rows<E, D, false>(dv, dvb, p.dvs[2], key, p.Nkv, 1.f, nullptr, nullptr, 0, h);
-  store_grad_rows<E, D, ROPE>(dk, dkb, p.dks[2], key, p.Nkv, p.scale, p.cos, p.sin, p.rs[0], h);
+  // the closing barrier of the last step ended every read of the stages
+  uint16_t* const wl = lds + w * 32 * D;
+  store_grad_rows<E, D, false>(wl, dv, dvb, p.dvs[2], n0w, key, p.Nkv, 1.f, nullptr, nullptr, 0, h);
+  store_grad_rows<E, D, ROPE>(wl, dk, dkb, p.dks[2], n0w, key, p.Nkv, p.scale, p.cos, p.sin, p.rs[0], h);
 }
 
 // ---------------------------------------------------------------------------
@@ -1028,8 +1020,9 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams& p, uint16_t* lds, i
     if (qrow < p.Nq) store_partial_row<D>(dq, p.part_dq + (((int64_t)bs_slot * BH + bh) * BMq + (qrow - m0)) * D, h);
     return;
   }
-  store_grad_rows<E, D, ROPE>(dq, p.dq + b * p.dqs[0] + hq * p.dqs[1], p.dqs[2], qrow, p.Nq, p.scale, p.cos,
-                              p.sin, p.rs[0], h);
+  // the closing barrier of the last step ended every read of the stages
+  store_grad_rows<E, D, ROPE>(lds + w * 32 * D, dq, p.dq + b * p.dqs[0] + hq * p.dqs[1], p.dqs[2], q0w, qrow, p.Nq,
+                              p.scale, p.cos, p.sin, p.rs[0], h);
 }
 
 // ---------------------------------------------------------------------------

@@ -202,28 +202,9 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 
   const float c2 = p.scale * kLog2e;
 
-  // ---- Q fragment (B operand of S^T = K Q^T), rotated once -------------
-  // The rotated q~ is rounded to 16 bits unscaled, as the reference kernel
-  // rounds it (attnfuse/compiler/codegen.py:126-135); the softmax scale is
-  // applied to the fp32 scores.
+  // Q fragment (B operand of S^T = K Q^T), filled once the first K/V tiles
+  // are on their way
   u32x4 qf[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    qf[ks] = (qrow < p.Nq) ? ld16(qbase + qrow * p.qs[2] + 16 * ks + 8 * h)
-                           : u32x4{0, 0, 0, 0};
-  }
-  if constexpr (ROPE) {
-    if (qrow < p.Nq) {
-      const uint16_t* cr = p.cos + qrow * rstr;
-      const uint16_t* sr = p.sin + qrow * rstr;
-#pragma unroll
-      for (int ks = 0; ks < KS / 2; ++ks) {
-        const int dl = 16 * ks + 8 * h, dh = dl + D / 2;
-        rope_pair<E>(qf[ks], qf[ks + KS / 2], ld16(cr + dl), ld16(sr + dl),
-                     ld16(cr + dh), ld16(sr + dh));
-      }
-    }
-  }
 
   // ---- key-tile schedule ------------------------------------------------
   int n_lo = 0, n_hi = p.Nkv, ntiles;
@@ -822,6 +803,28 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
     if constexpr (!kDefer) load_v(0, 0);
   }
   if (!kUnpiped && ntiles > 1) load_k(1, 1);
+  // The workgroup's query rows, rotated once.  The rotated q~ is rounded to 16
+  // bits unscaled, as the reference kernel rounds it
+  // (attnfuse/compiler/codegen.py:126-135); the softmax scale is applied to
+  // the fp32 scores.  Rotated before the first tiles' loads were issued, the
+  // rows held those loads up for a round trip to memory.
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    qf[ks] = (qrow < p.Nq) ? ld16(qbase + qrow * p.qs[2] + 16 * ks + 8 * h)
+                           : u32x4{0, 0, 0, 0};
+  }
+  if constexpr (ROPE) {
+    if (qrow < p.Nq) {
+      const uint16_t* cr = p.cos + qrow * rstr;
+      const uint16_t* sr = p.sin + qrow * rstr;
+#pragma unroll
+      for (int ks = 0; ks < KS / 2; ++ks) {
+        const int dl = 16 * ks + 8 * h, dh = dl + D / 2;
+        rope_pair<E>(qf[ks], qf[ks + KS / 2], ld16(cr + dl), ld16(sr + dl),
+                     ld16(cr + dh), ld16(sr + dh));
+      }
+    }
+  }
   wait_lds_dma();
   __syncthreads();
   f32x16 sa[BN / 32], sb[BN / 32];
@@ -995,18 +998,13 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
     return;
   }
   const float inv = (lt == 0.f) ? 1.f : 1.f / lt;
+#pragma unroll
+  for (int db = 0; db < DB; ++db) o[db] *= inv;
+  // every wave is past its last read of the tiles (the deferred P V of the
+  // last tile follows the loop's closing barrier)
+  if constexpr (kDefer) __syncthreads();
+  store_rows_via_lds<E, D>(lds + w * 32 * D, o, p.o + b * p.os[0] + hq * p.os[1], p.os[2], q0w, p.Nq);
   if (qre < p.Nq) {
-    uint16_t* orow = p.o + b * p.os[0] + hq * p.os[1] + (int64_t)qre * p.os[2];
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d0 = 32 * db + 8 * g + 4 * he;
-        u32x2 w2;
-        w2[0] = E::pack(o[db][4 * g] * inv, o[db][4 * g + 1] * inv);
-        w2[1] = E::pack(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv);
-        *reinterpret_cast<u32x2*>(orow + d0) = w2;
-      }
     if (p.lse != nullptr && he == 0) {
       float L = -INFINITY;
       if constexpr (NORM == NORM_SOFTMAX) {

@@ -78,15 +78,6 @@ inline int fwd_key_waves(int D, int mask, int64_t blocks32) {
   return blocks32 > most ? 0 : blocks32 <= most8 ? 8 : 4;
 }
 
-// Orders this wave's own LDS writes and reads of one tile, which no other
-// wave touches: a wave's LDS accesses complete in order, so this only holds
-// the compiler to the order.
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <class E, int D, bool ROPE, int KW>
 __global__ void __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2)))
     fwd_keys_kernel(const FwdKeysParams P) {
