@@ -198,3 +198,22 @@ def test_decode_ragged_splits_and_alibi(splits):
     sl = _alibi_slopes(Hq, "cpu", "torch.float32")
     want = O.naive_attention(Q.cpu(), K.cpu(), V.cpu(), alibi_slopes=sl, query_offset=N - 1)
     assert (out.cpu() - want).abs().max().item() <= TOL
+
+
+@pytest.mark.parametrize("splits", [1, 5])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_decode_one_query_head_per_kv_head(D, splits):
+    """The variant for one query head per key/value head, with ALiBi, a
+    ragged cache and an unsplit one."""
+    from attnfuse.runtime.dispatch import _alibi_slopes
+    from attnfuse.runtime.flash_decode import run_flash_decode
+    B, H, N = 2, 5, 1003
+    Q, K, V = _decode_inputs(B, H, H, N, D, seed=D)
+    fn = af.attention(lambda Q, K, V: af.softmax(af.alibi(af.scaled_dot_product(Q, K), H)) @ V)
+    g = fn(Q, K, V, return_graph=True)
+    out = torch.empty_like(Q)
+    run_flash_decode(g, Q, K, V, D ** -0.5, 1, H, out, num_splits=splits)
+    torch.cuda.synchronize()
+    sl = _alibi_slopes(H, "cpu", "torch.float32")
+    want = O.naive_attention(Q.cpu(), K.cpu(), V.cpu(), alibi_slopes=sl, query_offset=N - 1)
+    assert (out.cpu() - want).abs().max().item() <= TOL
