@@ -328,7 +328,7 @@ __device__ __forceinline__ void bwd_dq_f32_body(const BwdParams& p, int mask, in
   const int col = lane & 31, h = lane >> 5;
   const int nbh = p.B * p.Hq;
   int mb = wg / nbh;
-  const int bh = wg % nbh;
+  const int bh = xcd_head(wg % nbh, nbh);
   if (mask == MASK_CAUSAL || mask == MASK_CSW) mb = p.n_qblocks - 1 - mb;
   const int b = bh / p.Hq, hq = bh % p.Hq, hk = hq / p.G;
   const int qw0 = mb * BLK;  // first query of the workgroup

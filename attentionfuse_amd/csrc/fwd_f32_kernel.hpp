@@ -131,7 +131,7 @@ __global__ void __launch_bounds__((KW > 1 ? KW : kF32Waves) * 64) fwd_f32_kernel
   const int col = lane & 31, h = lane >> 5;
   const int nbh = p.B * p.Hq;
   int mb = (int)(blockIdx.x / nbh);
-  const int bh = (int)(blockIdx.x % nbh);
+  const int bh = xcd_head((int)(blockIdx.x % nbh), nbh);
   // causal-type masks: the longest key ranges first
   if (mask == MASK_CAUSAL || mask == MASK_CSW) mb = p.n_mblocks - 1 - mb;
   const int b = bh / p.Hq, hq = bh % p.Hq, hk = hq / p.G;
