@@ -345,8 +345,7 @@ int plan_decode(const af_decode_args* a, size_t max_ws, DecodeParams* out, size_
   if (a->key.bias == AF_BIAS_ALIBI && a->alibi_slopes == nullptr) return fail(AF_ERR_BAD_ARG, "ALiBi needs slopes");
   const int D = a->key.head_dim;
   int S = a->num_splits > 0 ? a->num_splits
-                            : af_decode_num_splits(a->batch, a->heads_q, a->heads_kv, a->seqlen_kv,
-                                                   a->key.dtype == AF_F32 ? 4 * D : D);
+                            : af_decode_num_splits(a->batch, a->heads_q, a->heads_kv, a->seqlen_kv, D);
   // split length rounded up to 32 keys; empty trailing splits are dropped
   int split_len = 0;
   auto trim = [&]() {
@@ -546,29 +545,26 @@ size_t af_fwd_blocksparse_workspace_bytes(const af_fwd_args* a, const af_blockma
   return a == nullptr ? 0 : bs_fwd_workspace(*a, bm).total;
 }
 
-// The split count with the least estimated time.  One workgroup alone on its
-// CU streams 128-dim 16-bit keys at 13.2 ns each (8 groups, 4096 keys: 8
-// splits 59 us for 32768 keys); all together reach 5.8 TB/s, less where the
-// last round of workgroups leaves CUs idle (64 groups x 32768 keys: 384
-// workgroups 197.9 us, 256 184.7, 512 182.5); the two add in squares near the
-// crossover.  Each workgroup has its start and merge, and more than one split
-// adds the combine launch, 2 us, and the partials of each (320 groups x 1500
-// keys: 4 splits 50.7 us, 8 56.5).  The four waves take 128 keys a step, so a
-// split counts in whole steps (8 groups x 1024 keys: 8 splits 7.6 us, 4 9.2,
-// 1 13.8; x 256 keys: 1 split 6.2, 2 7.5; x 600 keys: 4 splits 8.2, 8 7.4).
-// fp32 callers pass four times the head dim: twice the bytes, on the VALU.
-int32_t af_decode_num_splits(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen_kv,
-                             int32_t head_dim) {
-  if (batch <= 0 || heads_q <= 0 || heads_kv <= 0 || seqlen_kv <= 0) return 1;
-  const int g = heads_q / heads_kv;
-  const double groups = (double)batch * heads_kv * ((g + 15) / 16);
-  const double keys = seqlen_kv, dims = head_dim > 0 ? head_dim : 128;
+// Split count of a decode call, from an estimate of its time.  One workgroup
+// alone on its CU streams 128-dim 16-bit keys at 13.2 ns each (8 groups, 4096
+// keys: 8 splits 59 us for 32768 keys); all together reach 5.8 TB/s, less
+// where the last round of workgroups leaves CUs idle (64 groups x 32768 keys:
+// 384 workgroups 197.9 us, 256 184.7, 512 182.5); the two add in squares near
+// the crossover.  Each workgroup has its start and merge, and more than one
+// split adds the combine launch, 2 us, and the partials of each (320 groups x
+// 1500 keys: 4 splits 50.7 us, 8 56.5).  The four waves take 128 keys a step,
+// so a split counts in whole steps (8 groups x 1024 keys: 8 splits 7.6 us, 4
+// 9.2, 1 13.8; x 256 keys: 1 split 6.2, 2 7.5; x 600 keys: 4 splits 8.2, 8
+// 7.4).  fp32 callers pass four times the head dim: twice the bytes, on the
+// VALU.
+static double decode_rounds(double per_cu) { return per_cu < 1 ? 1 : std::ceil(per_cu) / per_cu; }
+
+static int decode_best_splits(double groups, double keys, double dims) {
   const double bw = groups * keys * dims * 4 / 5.8e6;                  // us
-  const int most = std::max(1, std::min(256, seqlen_kv / 96));
   int best = 1;
   double best_t = 0;
-  for (int s = 1; s <= most; s += s < 16 ? 1 : s < 64 ? 4 : 16) {
-    const double per_cu = groups * s / 256, rounds = per_cu < 1 ? 1 : std::ceil(per_cu) / per_cu;
+  for (int s = 1; s <= 256; s += s < 16 ? 1 : s < 64 ? 4 : 16) {
+    const double per_cu = groups * s / 256, rounds = decode_rounds(per_cu);
     const double one = 13.2e-3 * dims * std::ceil(keys / s / 128) * std::ceil(per_cu / 2);
     const double t = std::sqrt(one * one + bw * bw * rounds * rounds) + 0.2 * per_cu + (s > 1 ? 2.0 + 0.05 * s : 0.0);
     if (s == 1 || t < best_t) {
@@ -577,6 +573,37 @@ int32_t af_decode_num_splits(int32_t batch, int32_t heads_q, int32_t heads_kv, i
     }
   }
   return best;
+}
+
+// The count must not fall as the cache grows: a workspace sized for the
+// longest cache serves the shorter ones.  The least estimated time at each
+// length does not have that property (8 groups of 128 dims: 32 splits at 4500
+// keys, 18 at 4608), so the estimate picks the count of a long cache and the
+// length at which splitting begins to pay; between the two a split keeps 96
+// keys or more (most of a step; 256 at head dim 32, whose steps are short) in
+// whole rounds of workgroups, and more where every CU has a group already (320
+// groups x 1500 keys: 4 splits 41.2 us, 8 45.1, 2 43.7).  That is within 2 % of
+// the least estimate on average over lengths and head counts.
+int32_t af_decode_num_splits(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seqlen_kv,
+                             int32_t head_dim) {
+  if (batch <= 0 || heads_q <= 0 || heads_kv <= 0 || seqlen_kv <= 0) return 1;
+  const int g = heads_q / heads_kv;
+  const double groups = (double)batch * heads_kv * ((g + 15) / 16);
+  const double dims = head_dim > 0 ? head_dim : 128;
+  int fill = decode_best_splits(groups, 32768, dims);
+  if (seqlen_kv >= 65536) return std::max(fill, decode_best_splits(groups, 131072, dims));
+  if (fill == 1) return 1;
+  // the length from which the time saved per key pays for the combine, the
+  // partials and the part of a step a split wastes
+  const double cu1 = groups / 256, cuf = groups * fill / 256;
+  const double key = 13.2e-3 * dims / 128 * std::ceil(cu1 / 2), bw = groups * dims * 4 / 5.8e6;
+  const double gain = std::hypot(key, bw * decode_rounds(cu1)) - std::hypot(key / fill, bw * decode_rounds(cuf));
+  const double cost = 2.0 + 0.05 * std::min(fill, 8) + 0.6 * 13.2e-3 * dims + 0.2 * (std::min(cuf, cu1 + 2) - cu1);
+  if (gain <= 0 || seqlen_kv * gain < cost) return 1;
+  const double least = cu1 > 1 ? 256 * cu1 : dims < 64 ? 256 : 96;
+  const int s = std::max(1, (int)(seqlen_kv / least));
+  if (s >= fill) return fill;
+  return cu1 <= 1 && s * groups > 256 ? std::max(1, (int)(256 * std::floor(s * groups / 256) / groups)) : s;
 }
 
 size_t af_decode_workspace_bytes(int32_t batch, int32_t heads_q, int32_t head_dim, int32_t num_splits) {

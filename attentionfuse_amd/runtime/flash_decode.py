@@ -72,7 +72,9 @@ def run_flash_decode(graph: Graph, Q: torch.Tensor, K: torch.Tensor,
     _, H_kv, N_kv, _ = K.shape
     if H_kv != num_heads_kv:
         raise ValueError("num_heads_kv does not match K")
-    S = num_splits or _pick_num_splits(B, H_q, N_kv, H_kv, _split_dims(Q))
+    # a caller's workspace was sized by the library's own count
+    S = num_splits or _pick_num_splits(
+        B, H_q, N_kv, H_kv, _split_dims(Q) if workspace is None else D)
     # the library may drop empty trailing splits; size for the request
     nbytes = int(N.lib().af_decode_workspace_bytes(B, H_q, D, S))
     ws = workspace if workspace is not None else decode_workspace(Q.device, nbytes)

@@ -207,6 +207,8 @@ typedef struct af_decode_args {
   int32_t num_splits; /* <= 0: library default (af_decode_num_splits) */
 } af_decode_args;
 
+/* Default split count; it never falls as seqlen_kv grows, so a workspace sized
+ * for the longest cache serves the shorter ones. */
 int32_t af_decode_num_splits(int32_t batch, int32_t heads_q, int32_t heads_kv,
                              int32_t seqlen_kv, int32_t head_dim);
 size_t af_decode_workspace_bytes(int32_t batch, int32_t heads_q,

@@ -148,3 +148,24 @@ def test_unsplit_and_many_splits_into_unaligned_rows(D, splits):
     want = O.naive_attention(Q.cpu(), K.cpu(), V.cpu())
     assert (out.float().cpu() - want).abs().max().item() <= TOL[dtype]
     assert not buf[..., 0].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("heads", [(8, 2), (12, 12)])
+def test_workspace_of_the_longest_cache_serves_shorter_ones(heads, dtype):
+    """Sized once by the library's count for the longest cache, used with the
+    default count at every length up to it."""
+    from attnfuse.runtime import _native as native
+    Hq, Hkv = heads
+    D, longest = 128, 9000
+    lib = native.lib()
+    S = lib.af_decode_num_splits(1, Hq, Hkv, longest, D)
+    ws = torch.empty(lib.af_decode_workspace_bytes(1, Hq, D, S), dtype=torch.uint8, device="cuda")
+    tol = TOL.get(dtype, 3e-5)
+    for N in (256, 700, 1056, 2304, 4500, longest):
+        Q, K, V = make(1, Hq, Hkv, N, D, dtype, seed=N)
+        out = torch.full_like(Q, float("nan"))
+        run_flash_decode(None, Q, K, V, D ** -0.5, 0, Hkv, out, workspace=ws)
+        want = O.naive_attention(Q.cpu(), K.cpu(), V.cpu())
+        err = (out.float().cpu() - want).abs().max().item()
+        assert err <= tol, (N, err)
