@@ -140,7 +140,7 @@ class Graph:
     v: TensorSym
     root: MatMulPV
     _signature: Optional[str] = field(default=None, repr=False)
-    _facts: Optional[dict] = field(default=None, repr=False)
+    _facts: Optional[dict] = field(default=None, init=False, repr=False)
 
     def fact(self, name: str, compute):
         """``compute(self)``, remembered under ``name``: like the signature, a

@@ -226,5 +226,9 @@ def pack_strides(args, *tensors) -> None:
     at = type(args).q_stride.offset
     for i in range(0, len(tensors), 4):
         a, b, c, d = tensors[i:i + 4]
-        _pack16(args, at + 32 * i, *a.stride(), *b.stride(), *c.stride(),
-                *d.stride())
+        try:
+            _pack16(args, at + 32 * i, *a.stride(), *b.stride(),
+                    *c.stride(), *d.stride())
+        except struct.error:
+            raise ValueError("expected 4-D tensors, got "
+                             f"{[t.dim() for t in (a, b, c, d)]}") from None

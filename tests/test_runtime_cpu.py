@@ -158,3 +158,41 @@ def test_slopes_for_the_kernels_are_the_rounded_ones(dtype):
         got = _alibi_slopes_f32(H, torch.device("cpu"), dtype)
         assert got.dtype == torch.float32
         assert torch.equal(got, _alibi_slopes(H, "cpu", str(dtype)).float())
+
+
+@pytest.mark.parametrize("dims", [32, 64, 128, 256, 512])
+def test_default_splits_never_fall_as_the_cache_grows(dims):
+    """A decode workspace sized for the longest cache serves every shorter
+    one with the default split count."""
+    from attentionfuse_amd.runtime import _native as N
+    f = N.lib().af_decode_num_splits
+    for groups in (1, 3, 8, 11, 24, 64, 84, 192, 257, 320, 1000):
+        prev = 1
+        for n in [*range(1, 8192, 32), *range(8192, 140000, 512)]:
+            s = f(groups, 1, 1, n, dims)
+            assert prev <= s <= 256, (groups, n)
+            prev = s
+
+
+def test_remembered_facts_stay_out_of_copies():
+    """What a graph remembers of itself is not part of it."""
+    import dataclasses
+    import pickle
+    import attentionfuse_amd.runtime.backward as bwd
+
+    @af.attention
+    def causal(Q, K, V):
+        return af.softmax(af.causal(af.scaled_dot_product(Q, K))) @ V
+
+    t = torch.zeros(1, 1, 8, 64)
+    a = causal(t, t, t, return_graph=True)
+    assert bwd.can_backward(a) and a._facts
+    assert dataclasses.replace(a)._facts is None
+    assert bwd.can_backward(pickle.loads(pickle.dumps(a)))
+
+
+def test_strides_of_a_tensor_of_another_rank_are_refused():
+    from attentionfuse_amd.runtime import _native as N
+    t = torch.zeros(1, 2, 8, 64)
+    with pytest.raises(ValueError):
+        N.pack_strides(N.FwdArgsC(), t, t, t, t[0])
